@@ -34,8 +34,8 @@ import sys
 
 import torch
 
-_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-_PKG = os.path.join(_ROOT, "flashinfer-repo_amd")
+# the package of the tree that is the working folder
+_PKG = os.path.join(os.getcwd(), "flashinfer-repo_amd")
 if _PKG not in sys.path:
     sys.path.insert(0, _PKG)
 
