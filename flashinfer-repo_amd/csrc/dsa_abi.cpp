@@ -504,6 +504,7 @@ int dsa_indexer_topk(const dsa_indexer_args *a, void *stream) {
     p.k_num_pages = (int32_t)a->k_num_pages;
   }
   p.scores = a->scores_out ? a->scores_out : reinterpret_cast<float *>(ws + lay.scores);
+  p.want_scores = a->scores_out != nullptr;
   const hipError_t e = dsa::launch_indexer(p, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(DSA_ELAUNCH, "%s: launch failed: %s", fn, hipGetErrorString(e));
   return ok();
@@ -556,7 +557,9 @@ int dsa_indexer_prepare_k(const dsa_indexer_k_prepare_args *a, void *stream) {
   const int64_t b0 = a->first_position / 16, b1 = (a->first_position + a->count + 15) / 16;
   p.k_block0 = (int32_t)b0;
   p.k_blocks = (int32_t)(b1 - b0);
-  const hipError_t e = dsa::launch_indexer_prepare_k(p, static_cast<hipStream_t>(stream));
+  p.k_codes = reinterpret_cast<uint8_t *>(p.k_pieces) + dsa::kKPlaneCodeOffset;
+  p.k_code_stride = dsa::kKPlaneBlockBytes;
+  const hipError_t e = dsa::launch_indexer_prepare_k(p, dsa::kPrepPlanes, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(DSA_ELAUNCH, "%s: launch failed: %s", fn, hipGetErrorString(e));
   return ok();
 }

@@ -108,10 +108,10 @@ int set_error(int code, const char *msg);
 size_t attn_split_workspace(int64_t T, int64_t H, int64_t K, int32_t requested);
 
 // Lightning indexer.  Workspace layout (see indexer_workspace_layout):
-//   k_pieces [ceil(S/16)][3 pieces][2 k-steps][1024 B]  MFMA B operands, lane order
-//   k_max    [ceil(S/16)]                               max |value * 2^9| per block
-//   k_cs     [S] fp32                                   c_s = fl32(k_scale * 2^-18) per position
-//   scores   [T][S] fp32                                (unless the caller's)
+//   k_pieces [ceil(S/16)][6144 B]  piece planes p0, p1 (MFMA B operands, lane order), codes
+//   k_max    [ceil(S/16)]          max |value * 2^9| and max |c_s| |k_s| per block
+//   k_cs     [S] fp32              c_s = fl32(k_scale * 2^-18) per position
+//   scores   [T][S] fp32           (unless the caller's)
 struct IndexerParams {
   const uint8_t *q;       // [T][Hi][128] e4m3 codes
   const uint8_t *k;       // [S][128] e4m3 codes (or null: paged cache below)
@@ -132,8 +132,14 @@ struct IndexerParams {
   int32_t page_size;
   int32_t *out;           // [T][topk]
   float *scores;          // [T][S] (workspace or caller buffer)
-  int8_t *k_pieces;
-  int32_t *k_max;
+  int8_t *k_pieces;       // a block's planes p0, p1 (2 KB each), then its codes or third plane
+  int32_t *k_max;         // per block: largest |x|, and largest |c_s| |k_s| (packed)
+  uint8_t *k_codes;       // codes of block b at b * k_code_stride, 128 B per position, no NaN codes
+  int32_t k_code_stride;
+  int32_t want_scores;    // the caller reads the scores
+  int32_t estimated;      // the scores buffer holds estimates (set by the launcher)
+  int32_t est_fused;      // the estimate kernel prepares K (set by the launcher)
+  int32_t est_pairs, est_blocks;  // estimate kernel's split (set by its launcher)
   int32_t blocks_per_wg;  // 16-position blocks one score workgroup walks (set by the launcher)
   // k blocks the prep kernel derives planes for: [k_block0, k_block0 + k_blocks)
   // (0 blocks when the call reads prepared K planes)
@@ -151,8 +157,23 @@ IndexerWorkspace indexer_workspace_layout(int64_t T, int64_t Hi, int64_t S, bool
                                           bool own_k);
 
 hipError_t launch_indexer(const IndexerParams &p, hipStream_t stream);
-// Only the k planes of blocks [k_block0, k_block0 + k_blocks) (K preparation).
-hipError_t launch_indexer_prepare_k(const IndexerParams &p, hipStream_t stream);
+// The K preparation of blocks [k_block0, k_block0 + k_blocks): c_s and k_max, and
+enum KPrep {
+  kPrepCodes,   // the codes (a selection from estimates)
+  kPrepPlanes,  // planes p0 and p1 and the codes (prepared planes)
+  kPrepDiff,    // planes p0 and p1 and the third plane (exact scores)
+};
+hipError_t launch_indexer_prepare_k(const IndexerParams &p, KPrep what, hipStream_t stream);
+// Whether a selection without scores can run from estimates.
+bool estimates_apply(const IndexerParams &p);
+// Whether the estimate kernel prepares an unprepared call's K on its way.
+bool estimates_prepare_k(const IndexerParams &p);
+hipError_t launch_estimates(const IndexerParams &p, hipStream_t stream);
+// Selection of every row from p.scores (exact, or estimates).
+hipError_t launch_topk(const IndexerParams &p, hipStream_t stream);
+
+// Bytes of one 16-position block of the K planes, and the codes' place in it.
+constexpr int kKPlaneBlockBytes = 6144, kKPlaneCodeOffset = 4096;
 
 // Prepared K planes (dsa_indexer_prepare_k): the K half of the workspace
 // layout, [k_pieces][k_max][k_cs] of S positions, 256-byte aligned regions.

@@ -24,7 +24,8 @@ BUILD_DIR = os.path.join(os.path.dirname(PKG_DIR), "_build")
 LIB_PATH = os.path.join(PKG_DIR, "libdsa_amd.so")
 SAN_LIB_PATH = os.path.join(PKG_DIR, "libdsa_amd_san.so")
 
-SOURCES = ["dsa_abi.cpp", "dsa_attention.hip", "dsa_indexer.hip", "dsa_noalloc.hip"]
+SOURCES = ["dsa_abi.cpp", "dsa_attention.hip", "dsa_indexer.hip", "dsa_select.hip",
+           "dsa_noalloc.hip"]
 # host-side C-ABI code: validation, launch configuration, scratch-array setup
 HOST_ABI_SOURCES = ["dsa_abi.cpp", "dsa_noalloc.hip"]
 

@@ -228,9 +228,11 @@ int dsa_attn_merge(const dsa_attn_merge_args *args, void *stream);
  *   optional (NULL = not returned; masked entries hold -inf).
  * head_dim must be 128, num_heads 16, 32, 48 or 64, topk <= 2^24.  The
  * workspace (dsa_indexer_workspace_bytes, 256-byte aligned) holds the MFMA
- * operand pieces of k and, unless scores_out is given, the scores (the q
- * operands are derived inside the score kernel); a call whose workspace
- * size is 0 may pass NULL.
+ * operand pieces of k and, unless scores_out is given, the scores or their
+ * estimates (a selection whose scores are not returned computes exact scores
+ * only where estimates, proven to lie within a bound of them, leave the
+ * choice open: the same sets); a call whose workspace size is 0 may pass
+ * NULL.
  */
 typedef struct dsa_indexer_args {
   const uint8_t *q_idx;
@@ -276,9 +278,9 @@ int dsa_indexer_topk(const dsa_indexer_args *args, void *stream);
  * Prepared K planes (no counterpart in the reference, whose score kernel
  * re-reads and dequantises K on every call, indexer_kernel.py:185-275).  The
  * K cache changes only where tokens are appended, so the MFMA operand planes
- * the score kernel reads (per 16-position block: the e4m3 values as signed
- * 7-bit pieces in MFMA lane order, the block's largest magnitude, and
- * fl32(k_scale * 2^-18) per position) can be derived once and kept beside
+ * the score kernels read (per 16-position block: the e4m3 values as signed
+ * 7-bit pieces in MFMA lane order and as codes, the block's largest magnitude
+ * and row norm, and fl32(k_scale * 2^-18) per position) can be derived once and kept beside
  * the cache.  dsa_indexer_prepare_k (re)derives the blocks that hold
  * positions [first_position, first_position + count) of a sequence of
  * num_positions positions (flat k_idx/k_scale, or a paged K cache read

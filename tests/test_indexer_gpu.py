@@ -535,3 +535,123 @@ def test_planes_in_graph_replays_match_eager():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+
+
+# ---- selection without scores: estimates, exact where they leave it open ---
+
+def _select_both(d, topk, block_table=None):
+    """The selection of the call that returns no scores (estimates, and exact
+    scores of the positions those leave open) and of the call that computes
+    every exact score, whose scores and sets the tests above compare with the
+    oracle."""
+    g = workloads.to_device(d, DEV)
+    args = (g["q_idx"], g["k_idx"], g["k_scale"], g["weights"], g["causal_limit"], topk)
+    got = run_indexer_and_topk(*args)
+    want, _ = run_indexer_and_topk(*args, return_scores=True)
+    torch.cuda.synchronize()
+    return got.cpu().numpy(), want.cpu().numpy()
+
+
+def _full_range(d, g):
+    """q and K codes over the whole e4m3 range (rows quantised by their largest
+    magnitude, as k_append does)."""
+    T, Hi, _ = d["q_idx"].shape
+    q, k = torch.randn(T, Hi, 128, generator=g), torch.randn(d["k_idx"].shape[0], 128, generator=g)
+    qs, ks = (x.abs().amax(-1, keepdim=True) / 448.0 for x in (q, k))
+    return dict(d, q_idx=workloads.e4m3(q / qs), k_idx=workloads.e4m3(k / ks), k_scale=ks[:, 0].contiguous(),
+                weights=d["weights"] * qs[..., 0])
+
+
+# S around the register top-k's sizes and the 16-position blocks, top-k next to 1
+# and to the row length, token counts around the pairs and fours of the waves
+@pytest.mark.parametrize("T,Hi,S,topk", [(1, 64, 65, 64), (2, 16, 8192, 2048), (3, 32, 8193, 1), (5, 48, 16384, 2048),
+                                         (7, 64, 16385, 16000), (9, 64, 32768, 2048), (6, 16, 32751, 2047),
+                                         (33, 64, 2049, 2048)])
+@pytest.mark.parametrize("full_range", [False, True])
+def test_selection_without_scores_matches_oracle(T, Hi, S, topk, full_range):
+    gen = torch.Generator().manual_seed(S + T)
+    d = workloads.indexer_inputs(T=T, Hi=Hi, S=S, seed=T * 31 + S)
+    if full_range:
+        d = _full_range(d, gen)
+    lim = d["causal_limit"].clone()
+    lim[0] = S - 1
+    if T > 2:
+        lim[1], lim[2] = S // 2, topk  # one candidate more than are taken
+    d["causal_limit"] = lim
+    print(f"select T={T} Hi={Hi} S={S} k={topk} full_range={full_range}", flush=True)
+    got, want = _select_both(d, topk)
+    ref, _ = _oracle(d, topk)
+    for t in range(T):
+        assert np.array_equal(np.sort(got[t]), np.sort(ref[t])), f"row {t} set differs from the oracle"
+    assert np.array_equal(got, want)
+
+
+def _hard(kind, T, Hi, S):
+    gen = torch.Generator().manual_seed(len(kind) * 1000 + S)
+    d = workloads.indexer_inputs(T=T, Hi=Hi, S=S, seed=17 + S)
+    d["causal_limit"] = torch.full((T,), S - 1, dtype=torch.int32)
+    k = d["k_idx"].view(torch.float8_e4m3fn).float()
+    if kind == "many equal rows":         # more open positions than are ranked
+        k = k[torch.randint(0, 3, (S,), generator=gen)]
+        d["k_scale"] = torch.ones(S)
+    elif kind == "nearly equal rows":     # scores apart by less than the estimate's error
+        k = k[:1].expand(S, 128).clone()
+        k[torch.arange(S), torch.randint(0, 128, (S,), generator=gen)] = 2.0 ** -9
+        d["k_scale"] = 1.0 + torch.arange(S).float()[torch.randperm(S, generator=gen)] * 2.0 ** -23
+    elif kind == "outlier rows":
+        k[torch.rand(S, generator=gen) < 0.05] *= 8
+    elif kind == "outlier scales":
+        d["k_scale"][::97] *= 2.0 ** 20
+        d["k_scale"][5::97] *= -1.0
+    elif kind == "zero rows":
+        k[torch.rand(S, generator=gen) < 0.7] = 0.0
+    elif kind == "wide exponents":
+        k *= torch.exp2(torch.randint(-9, 9, (S, 128), generator=gen).float())
+    elif kind == "zero weights":
+        d["weights"][::2] = 0.0
+    elif kind == "tiny weights":
+        d["weights"] *= 1e-30
+        d["weights"][0] *= 1e-12          # subnormal products
+    elif kind == "huge weights":
+        d["weights"] *= 1e30              # the exact sum overflows
+    elif kind == "weights not finite":
+        d["weights"][0, 3], d["weights"][1, 0], d["weights"][2, 5] = float("inf"), float("nan"), -float("inf")
+    elif kind == "scales not finite":
+        d["k_scale"][[3, 700]] = float("inf")
+        d["k_scale"][[44, 800]] = float("nan")
+        d["k_scale"][[45, 900]] = -float("inf")
+    d["k_idx"] = workloads.e4m3(k.clamp(-448, 448))
+    if kind == "NaN codes":               # count as zeros in q and k
+        d["k_idx"] = d["k_idx"].clone()
+        d["k_idx"].view(-1)[torch.randint(0, S * 128, (S * 8,), generator=gen)] = 0x7F
+        d["k_idx"][100:200, 5] = 0xFF
+        d["q_idx"] = d["q_idx"].clone()
+        d["q_idx"][:, ::3, 7] = 0xFF
+    return d
+
+
+@pytest.mark.parametrize("S", [6000, 20000])
+@pytest.mark.parametrize("kind", ["many equal rows", "nearly equal rows", "outlier rows", "outlier scales", "zero rows",
+                                  "wide exponents", "zero weights", "tiny weights", "huge weights",
+                                  "weights not finite", "scales not finite", "NaN codes"])
+def test_selection_without_scores_of_hard_rows(kind, S):
+    """Rows whose estimates leave many positions open or whose error bound is
+    not safe take exact scores for the whole row; codes, weights and scales
+    at the ends of their formats."""
+    d = _hard(kind, 4, 32, S)
+    print(f"hard rows: {kind} S={S}", flush=True)
+    for topk in (300, 2048):
+        got, want = _select_both(d, topk)
+        assert np.array_equal(got, want), kind
+
+
+def test_selection_without_scores_after_nan_filled_lds():
+    d = _full_range(workloads.indexer_inputs(T=5, Hi=64, S=20000, seed=77), torch.Generator().manual_seed(78))
+    ref, _ = _oracle(d, 2048)
+    g = workloads.to_device(d, DEV)
+    for r in range(3):
+        fill_lds_with_nan(DEV)
+        print(f"NaN-filled LDS selection call {r}", flush=True)
+        out = run_indexer_and_topk(g["q_idx"], g["k_idx"], g["k_scale"], g["weights"], g["causal_limit"], 2048)
+        torch.cuda.synchronize()
+        assert np.array_equal(np.sort(out.cpu().numpy(), axis=1), np.sort(ref, axis=1))
