@@ -79,9 +79,10 @@ __device__ __forceinline__ uint32_t norm_bits_up(uint32_t bits) {  // of a non-n
   return min((bits + 0x1ffffu) >> 17, 0x3fffu);
 }
 // |c_s| |k_s| of a position whose codes' squares sum to n2 (the factor covers
-// the sum's and the root's rounding).
+// the sum's and the root's rounding; 0 only if either is).
 __device__ __forceinline__ uint32_t position_norm_bits(float cs, float n2) {
-  return norm_bits_up(__float_as_uint(fabsf(cs) * sqrtf(n2) * 1.001f));
+  const uint32_t tiny = cs != 0.f && n2 > 0.f ? 1u : 0u;
+  return norm_bits_up(max(__float_as_uint(fabsf(cs) * sqrtf(n2) * 1.001f), tiny));
 }
 __device__ __forceinline__ float norm_from_bits(uint32_t b14) { return __uint_as_float(b14 << 17); }
 

@@ -140,6 +140,7 @@ struct IndexerParams {
   int32_t estimated;      // the scores buffer holds estimates (set by the launcher)
   int32_t est_fused;      // the estimate kernel prepares K (set by the launcher)
   int32_t est_pairs, est_blocks;  // estimate kernel's split (set by its launcher)
+  int32_t chunk, n_chunks, list_len, list_shift;  // long rows' chunks and lists (set by the launcher)
   int32_t blocks_per_wg;  // 16-position blocks one score workgroup walks (set by the launcher)
   // k blocks the prep kernel derives planes for: [k_block0, k_block0 + k_blocks)
   // (0 blocks when the call reads prepared K planes)

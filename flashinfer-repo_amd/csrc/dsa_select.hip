@@ -3,7 +3,8 @@
 //
 // Kernels:
 //   dsa_idx_estimate_kernel     every score within a proven bound, by bf16 MFMAs
-//   dsa_idx_topk_kernel         one workgroup per row, the row in registers
+//   dsa_idx_topk_kernel         from exact scores, up to 32768 positions: one
+//                               workgroup per row, the row in registers
 //                               (loaded coalesced, 1024-strided, through one
 //                               buffer descriptor): two radix passes (8 bits
 //                               each, histograms replicated 32 ways so equal
@@ -17,8 +18,12 @@
 //                               more passes.  The selection is a position
 //                               bitmap built from ballots; one scan turns it
 //                               into ranks in ascending position order.
+//   dsa_idx_topk_estimates_kernel  the same from estimates
+//   dsa_idx_topk_chunk_kernel,
+//   dsa_idx_topk_merge_kernel   rows longer than 32768 positions, from
+//                               estimates: a list per chunk, then the lists
 //   dsa_idx_topk_stream_kernel  a four-pass selection re-reading the row from
-//                               memory, for rows longer than 32768 positions.
+//                               memory: longer rows from exact scores
 #include <algorithm>
 #include <cstdint>
 #include <type_traits>
@@ -706,11 +711,12 @@ __device__ __forceinline__ void exact_scores(const IndexerParams &p, Shared &sh,
 // ---- the register top-k, one row per workgroup -----------------------------
 
 // Key e of thread tid is position e*1024 + tid (coalesced), so the 64 lanes of
-// a wave hold 64 consecutive positions of every e.  A buffer load over the row
-// needs one 32-bit offset register for all loads (kept in flight together).
+// a wave hold 64 consecutive positions of every e.  A buffer load over the
+// `len` scores needs one 32-bit offset register for all loads (kept in flight
+// together).
 template <int EPT>
-__device__ __forceinline__ void load_keys(const IndexerParams &p, const float *row, uint32_t (&key)[EPT]) {
-  const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(row), 0, p.S * 4, kBufferFlags);
+__device__ __forceinline__ void load_keys(const float *scores, int len, uint32_t (&key)[EPT]) {
+  const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(scores), 0, len * 4, kBufferFlags);
 #pragma unroll
   for (int e = 0; e < EPT; ++e)
     key[e] = __builtin_amdgcn_raw_buffer_load_b32(rs, threadIdx.x * 4, e * kTopkThreads * 4, 0);
@@ -726,14 +732,11 @@ __device__ __forceinline__ void clear_counts(Shared &sh) {
   if (threadIdx.x == 0) sh.n_cand = sh.n_above = 0;
 }
 
-// Scores to order keys and two radix passes: the k-th largest key lies in the
-// 16-bit bin `prefix`, and `need` of the bin's keys are among the k largest.
-// Adding +0.0 turns -0.0 into +0.0; the key orders the scores as unsigned
-// integers.  The keys past the n candidates become 0, the lowest, and are taken
-// out of the histograms.
-template <int EPT, typename Shared>
-__device__ __forceinline__ void find_bin(const IndexerParams &p, Shared &sh, int n, uint32_t (&key)[EPT],
-                                         uint32_t &prefix, uint32_t &mask, int &need) {
+// Scores to order keys.  Adding +0.0 turns -0.0 into +0.0; the key orders the
+// scores as unsigned integers.  The keys past the n candidates become 0, the
+// lowest, and are taken out of the histograms.
+template <int EPT>
+__device__ __forceinline__ void to_keys(int n, uint32_t (&key)[EPT]) {
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int full = max(0, n - wave * 64) / kTopkThreads;  // keys e below it are all candidates
@@ -743,10 +746,16 @@ __device__ __forceinline__ void find_bin(const IndexerParams &p, Shared &sh, int
     key[e] = u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
     if (e >= full && e * kTopkThreads + tid >= n) key[e] = kPhantomKey;  // the first test is uniform
   }
+}
+
+// Two radix passes: the k-th largest key lies in the 16-bit bin `prefix`, and
+// `need` of the bin's keys are among the k largest.
+template <int EPT, typename Shared>
+__device__ __forceinline__ void find_bin(const IndexerParams &p, Shared &sh, const uint32_t (&key)[EPT],
+                                         int phantom, uint32_t &prefix, uint32_t &mask, int &need) {
   prefix = 0;
   mask = 0;
   need = p.topk;
-  const int phantom = EPT * kTopkThreads - n;
 #pragma unroll 1
   for (int shift = 24; shift >= 16; shift -= 8)
     radix_pass_regs(sh, sh.hist[shift == 24 ? 0 : 1], true, shift, key, prefix, mask, need, phantom);
@@ -817,9 +826,11 @@ __device__ __forceinline__ void rank_open(Shared &sh, int n_open, int need) {
   __syncthreads();
 }
 
-// The marked positions (of the n candidates), or their slots, in ascending order.
-template <int KEYS, typename Shared>
-__device__ __forceinline__ void write_marked(const IndexerParams &p, Shared &sh, int t, int n, int32_t *out) {
+// The marked places (of the first n), as positions at(place) or their slots, in
+// ascending order.
+template <int KEYS, typename Shared, typename At>
+__device__ __forceinline__ void write_marked(const IndexerParams &p, Shared &sh, int t, int n, int32_t *out,
+                                             At at) {
   const int tid = threadIdx.x;
   const uint32_t *bits32 = (const uint32_t *)sh.bits;
   int unused;
@@ -843,7 +854,7 @@ __device__ __forceinline__ void write_marked(const IndexerParams &p, Shared &sh,
   for (int r0 = tid; r0 < p.topk; r0 += 4 * kTopkThreads) {
     int v[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = sh.pos[min(r0 + u * kTopkThreads, p.topk - 1)];
+    for (int u = 0; u < 4; ++u) v[u] = at(sh.pos[min(r0 + u * kTopkThreads, p.topk - 1)]);
     if (p.block_table != nullptr) {
       const int32_t *bt = p.block_table + (int64_t)t * p.bt_stride;
       int page[4];
@@ -858,11 +869,12 @@ __device__ __forceinline__ void write_marked(const IndexerParams &p, Shared &sh,
   }
 }
 
-// Selection of a row from its exact scores: the keys above the bin are taken,
-// those in it ranked, or, where many share it, two more passes pin the k-th key.
+// Marks the k largest of exact keys: the keys above the bin are taken, those in
+// it ranked, or, where many share it, two more passes pin the k-th key.  The
+// `phantom` keys past the first n are 0 (the lowest) and may be marked.
 template <int EPT, typename Shared>
-__device__ __forceinline__ void select_exact(const IndexerParams &p, Shared &sh, int t, int n,
-                                             uint32_t (&key)[EPT], int32_t *out) {
+__device__ __forceinline__ void mark_exact(const IndexerParams &p, Shared &sh, int n,
+                                           const uint32_t (&key)[EPT], int phantom) {
   constexpr int KEYS = EPT * kTopkThreads;
   constexpr int kWaves = kTopkThreads / 64;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -872,14 +884,13 @@ __device__ __forceinline__ void select_exact(const IndexerParams &p, Shared &sh,
   int need, unused;
   clear_counts(sh);
   __syncthreads();
-  find_bin(p, sh, n, key, prefix, mask, need);
+  find_bin(p, sh, key, phantom, prefix, mask, need);
   mark_taken(sh, n, key, prefix, prefix | 0xffffu, prefix | 0xffffu);
   __syncthreads();
   const int n_open = sh.n_cand;
   if (n_open <= kMaxSurvivors) {  // uniform
     rank_open(sh, n_open, need);
   } else {
-    const int phantom = KEYS - n;
     // Many keys share the bin: two more passes pin the k-th key itself;
     // keys above it are taken, and `need` of its ties, lowest positions first.
     need = sh.need;
@@ -907,95 +918,142 @@ __device__ __forceinline__ void select_exact(const IndexerParams &p, Shared &sh,
       eq &= eq - 1;
     }
     if (take != 0) bits32[tid] |= take;  // this thread's own word
+    __syncthreads();
   }
-  write_marked<KEYS>(p, sh, t, n, out);
+}
+
+// ---- the estimates' bound ---------------------------------------------------
+
+// Eight q codes of a row per thread, for the bound and the exact scores: 16
+// threads per head, heads in the order of the MFMA rows (q_operands).
+struct RowCodes {
+  int row, hb, head;  // MFMA row, head block and head
+  uint2 codes;
+  float w;  // the head's weight
+};
+__device__ __forceinline__ RowCodes load_row_codes(const IndexerParams &p, int t) {
+  const int tid = threadIdx.x;
+  RowCodes r;
+  r.row = (tid >> 4) & 15;
+  r.hb = tid >> 8;
+  r.head = (r.row >> 2) * (p.Hi >> 2) + 4 * r.hb + (r.row & 3);
+  r.codes = make_uint2(0, 0);
+  r.w = 0.f;
+  if (tid < p.Hi * 16) {
+    r.codes = *(const uint2 *)(p.q + ((int64_t)t * p.Hi + r.head) * kIdxDim + (tid & 15) * 8);
+    r.w = p.w[(int64_t)t * p.Hi + r.head];
+  }
+  return r;
+}
+
+// Whether any of the 16 threads' codes (a head's) is not zero.
+__device__ __forceinline__ bool row_any_code(uint2 codes) {
+  const bool any = ((drop_nan(codes.x) | drop_nan(codes.y)) & 0x7f7f7f7fu) != 0;
+  return ((__ballot(any) >> (threadIdx.x & 48)) & 0xffffu) != 0;
+}
+
+// Each wave's share of sum_h |w_h| |q_h| (four heads) and of max_s |c_s| |k_s|
+// over k_max blocks [blk0, blk1); the weights and the code table.  bound()
+// follows, behind a barrier.
+template <typename Shared>
+__device__ __forceinline__ void bound_shares(const IndexerParams &p, Shared &sh, const RowCodes &r, int blk0,
+                                             int blk1) {
+  constexpr int kWaves = kTopkThreads / 64;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint32_t kn = 0;
+  for (int b = blk0 + tid; b < blk1; b += kTopkThreads) kn = max(kn, (uint32_t)p.k_max[b] >> kMaxXBits);
+  float x = row_sum_last(sum_squares8(drop_nan(r.codes.x), drop_nan(r.codes.y)));
+  // (a product that is not zero counts as at least the smallest normal, so the
+  // sum is 0 only where every score is 0)
+  x = (lane & 15) == 15 ? __builtin_amdgcn_sqrtf(x) * fabsf(r.w) : 0.f;
+  const bool any = row_any_code(r.codes);
+  if ((lane & 15) == 15 && x == 0.f && r.w != 0.f && any) x = 0x1p-126f;
+  x = rows_sum_last(x);
+  const uint32_t m = wave_max_last(kn);
+  if (lane == 63) {
+    sh.q_part[wave] = x;
+    sh.k_part[wave] = m;
+  }
+  if (tid < p.Hi * 16 && (tid & 15) == 0) sh.w[r.head] = r.w;
+  if (wave >= kWaves - 4) sh.lut[tid & 255] = piece_word(tid & 255);
+}
+
+// 2 E into sh.band, or NaN where E is not a safe bound (by the last wave; read
+// behind a later barrier).  0: every exact score is 0, and so is its estimate.
+template <typename Shared>
+__device__ __forceinline__ void bound(Shared &sh) {
+  constexpr int kWaves = kTopkThreads / 64;
+  const int lane = threadIdx.x & 63;
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) != kWaves - 1) return;
+  const int i = min(lane, kWaves - 1);
+  const float x = row_sum_last(lane < kWaves ? sh.q_part[i] : 0.f);
+  const uint32_t m = wave_max_last(lane < kWaves ? sh.k_part[i] : 0u);
+  const float W = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), 15));
+  const float A = norm_from_bits(__builtin_amdgcn_readlane(m, 63)) * 0x1p18f, WA = W * A;
+  // no overflow on either side's way (the exact sum carries 2^18), no
+  // underflow that matters, no NaN
+  const bool safe = W > 0x1p-60f && W < 0x1p95f && A > 0x1p-60f && A < 0x1p60f && WA < 0x1p100f;
+  const bool zero = (W == 0.f && A < INFINITY) || (A == 0.f && W < INFINITY);
+  if (lane == 0)
+    sh.band = safe ? 2.f * kEstimateError * WA : zero ? 0.f : __uint_as_float(0x7fc00000u);
+}
+
+// The row's q pieces, in the histograms' place.
+template <typename Shared>
+__device__ __forceinline__ void store_row_pieces(const IndexerParams &p, Shared &sh, const RowCodes &r) {
+  if ((int)threadIdx.x < p.Hi * 16)
+    store_pieces8(sh.lut, sh.qp + r.hb * (6 * kChunk), r.row, (threadIdx.x & 15) * 8, r.codes);
 }
 
 // Top-k of one row per workgroup from exact scores.
 template <int EPT>
 __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_kernel(IndexerParams p) {
   static_assert(EPT <= 32, "one 32-bit bitmap word per thread at most");
-  __shared__ __attribute__((aligned(16))) TopkShared<EPT * kTopkThreads> sh;
+  constexpr int KEYS = EPT * kTopkThreads;
+  __shared__ __attribute__((aligned(16))) TopkShared<KEYS> sh;
   const int t = blockIdx.x;
   int32_t *out = p.out + (int64_t)t * p.topk;
   const int n = candidates(p, t);  // candidates 0..n-1
   if (take_all(p, t, out, n)) return;               // n > topk >= 1 below
   uint32_t key[EPT];
-  load_keys(p, p.scores + (int64_t)t * p.S, key);
-  select_exact(p, sh, t, n, key, out);
+  load_keys(p.scores + (int64_t)t * p.S, p.S, key);
+  to_keys(n, key);
+  mark_exact(p, sh, n, key, KEYS - n);
+  write_marked<KEYS>(p, sh, t, n, out, [](int i) { return i; });
 }
 
 // Top-k of one row per workgroup from estimates.  The exact k-th largest score
 // lies within E of the estimates' bin, so keys more than 2 E above the bin are
 // taken, those more than 2 E below it are not, and the exact scores of the ones
 // between (a few dozen of 32768 ordinary scores) are computed here and ranked.
-// Where E is not a safe bound (zero, huge or non-finite weights or scales) or
+// Where E is not a safe bound (huge, tiny or non-finite weights or scales) or
 // too many keys are open, the row's exact scores are computed and selected from.
 template <int EPT>
 __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_estimates_kernel(IndexerParams p) {
   constexpr int KEYS = EPT * kTopkThreads;
-  constexpr int kWaves = kTopkThreads / 64;
   __shared__ __attribute__((aligned(16))) TopkShared<KEYS> sh;
   const int t = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   float *row = p.scores + (int64_t)t * p.S;
   int32_t *out = p.out + (int64_t)t * p.topk;
-  // eight q codes per thread, for the bound and the exact scores: 16 threads
-  // per head, heads in the order of the MFMA rows (q_operands)
-  const int q_mc = (tid >> 4) & 15, q_hb = tid >> 8;
-  const int q_head = (q_mc >> 2) * (p.Hi >> 2) + 4 * q_hb + (q_mc & 3);
-  uint2 qc = make_uint2(0, 0);
-  float qw = 0.f;
-  uint32_t kn = 0;  // largest norm bits of this thread's blocks
-  if (tid < p.Hi * 16) {
-    qc = *(const uint2 *)(p.q + ((int64_t)t * p.Hi + q_head) * kIdxDim + (tid & 15) * 8);
-    qw = p.w[(int64_t)t * p.Hi + q_head];
-  }
+  const RowCodes rc = load_row_codes(p, t);
   uint32_t key[EPT];
-  load_keys(p, row, key);  // beside the load of the row's limit
+  load_keys(row, p.S, key);  // beside the load of the row's limit
   const int n = candidates(p, t);  // candidates 0..n-1
   if (take_all(p, t, out, n)) return;               // n > topk >= 1 below
 
-#pragma unroll
-  for (int j = 0; j < (KEYS / 16 + kTopkThreads - 1) / kTopkThreads; ++j) {
-    const int b = j * kTopkThreads + tid;
-    if (b < (n + 15) >> 4) kn = max(kn, (uint32_t)p.k_max[b] >> kMaxXBits);
-  }
   clear_counts(sh);
-  {
-    // the wave's share of sum_h |w_h| |q_h| (four heads) and of max_s |c_s| |k_s|
-    float x = row_sum_last(sum_squares8(drop_nan(qc.x), drop_nan(qc.y)));
-    x = (lane & 15) == 15 ? __builtin_amdgcn_sqrtf(x) * fabsf(qw) : 0.f;
-    x = rows_sum_last(x);
-    const uint32_t m = wave_max_last(kn);
-    if (lane == 63) {
-      sh.q_part[wave] = x;
-      sh.k_part[wave] = m;
-    }
-    if (tid < p.Hi * 16 && (tid & 15) == 0) sh.w[q_head] = qw;
-    if (wave >= kWaves - 4) sh.lut[tid & 255] = piece_word(tid & 255);
-  }
+  bound_shares(p, sh, rc, 0, (n + 15) >> 4);
   __syncthreads();
-  if (wave == kWaves - 1) {  // the bound, read after the passes
-    const int i = min(lane, kWaves - 1);
-    const float x = row_sum_last(lane < kWaves ? sh.q_part[i] : 0.f);
-    const uint32_t m = wave_max_last(lane < kWaves ? sh.k_part[i] : 0u);
-    const float W = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), 15));
-    const float A = norm_from_bits(__builtin_amdgcn_readlane(m, 63)) * 0x1p18f, WA = W * A;
-    // no overflow on either side's way (the exact sum carries 2^18), no
-    // underflow that matters, no NaN
-    const bool safe = W > 0x1p-60f && W < 0x1p95f && A > 0x1p-60f && A < 0x1p60f && WA < 0x1p100f;
-    if (lane == 0) sh.band = safe ? 2.f * kEstimateError * WA : __uint_as_float(0x7fc00000u);
-  }
+  bound(sh);
+  to_keys(n, key);
   uint32_t prefix, mask;
   int need;
-  find_bin(p, sh, n, key, prefix, mask, need);
+  find_bin(p, sh, key, KEYS - n, prefix, mask, need);
   const float band = sh.band;
   mark_taken(sh, n, key, order_key(key_value(prefix) - band),
              order_key(key_value(prefix | 0xffffu) + band), prefix | 0xffffu);
-  // the row's q pieces, in the histograms' place
-  if (tid < p.Hi * 16) store_pieces8(sh.lut, sh.qp + q_hb * (6 * kChunk), q_mc, (tid & 15) * 8, qc);
+  store_row_pieces(p, sh, rc);
   __syncthreads();
   const int n_open = sh.n_cand;
   if (band == band && n_open <= kMaxOpen) {  // uniform
@@ -1006,16 +1064,195 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_estimates_kernel(In
                  });
     // (the keys above the bin that are open are not taken for sure)
     rank_open(sh, n_open, need + sh.n_above);
-    write_marked<KEYS>(p, sh, t, n, out);
+    write_marked<KEYS>(p, sh, t, n, out, [](int i) { return i; });
     return;
   }
-  // every candidate's exact score, then the selection from those
-  exact_scores(p, sh, (n + 15) >> 4, [&](int b, int c) { return min(b * 16 + c, p.S - 1); },
-               [&](int b, int c, float v) {
-                 if (b * 16 + c < n) row[b * 16 + c] = v;
-               });
-  load_keys(p, row, key);
-  select_exact(p, sh, t, n, key, out);
+  // every candidate's exact score (estimates of zeros are), then the selection
+  // from those
+  if (!(band == 0.f)) {
+    exact_scores(p, sh, (n + 15) >> 4, [&](int b, int c) { return min(b * 16 + c, p.S - 1); },
+                 [&](int b, int c, float v) {
+                   if (b * 16 + c < n) row[b * 16 + c] = v;
+                 });
+    load_keys(row, p.S, key);
+    to_keys(n, key);
+  }
+  mark_exact(p, sh, n, key, KEYS - n);
+  write_marked<KEYS>(p, sh, t, n, out, [](int i) { return i; });
+}
+
+// ---- rows longer than the registers hold: chunks, then their lists ----------
+//
+// A row of p.n_chunks chunks: one workgroup per chunk lists the chunk's
+// positions that can be among the row's k largest -- those whose estimate is
+// within 2 E of the chunk's own k-th largest, or above -- and one workgroup per
+// row selects from the lists as the kernel above does from a row.  A list
+// takes the place of its chunk's estimates (all of a chunk's are in registers
+// by then): p.list_len order keys, 0 past the list's end, then their
+// positions, ascending.  A chunk whose bound is not safe, or whose list would
+// not fit, lists its k largest exact scores.  2 rows of 131071 positions, top-k
+// 2048: chunks 17 us, lists 20, against 235 for the four passes over exact
+// scores (one workgroup re-reading the row, its last pass uncoalesced).
+
+// The chunk's marked keys (of its first n places) as its list.
+template <int EPT, typename Shared>
+__device__ __forceinline__ void write_list(const IndexerParams &p, Shared &sh, int n, int c0,
+                                           const uint32_t (&key)[EPT], int total, float *list) {
+  constexpr int kWaves = kTopkThreads / 64;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int *rank = (const int *)sh.eqbits;  // first rank of each 32-place word
+  uint32_t *keys = (uint32_t *)list;
+  int32_t *places = (int32_t *)list + p.list_len;
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) {
+    const uint64_t m = sh.bits[e * kWaves + wave];
+    if (m != 0 && ((m >> lane) & 1)) {
+      const int o = rank[(e * kWaves + wave) * 2] +
+                    __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+      keys[o] = max(key[e], 1u);
+      places[o] = c0 + e * kTopkThreads + tid;
+    }
+  }
+  for (int i = total + tid; i < p.list_len; i += kTopkThreads) keys[i] = 0;
+}
+
+// Masks the marks to the first n places and ranks their words; returns how
+// many are marked.
+template <int KEYS, typename Shared>
+__device__ __forceinline__ int rank_marks(Shared &sh, int n) {
+  const int tid = threadIdx.x;
+  uint32_t *bits32 = (uint32_t *)sh.bits;
+  const int nw = n - tid * 32;
+  uint32_t sel = tid < KEYS / 32 ? bits32[tid] : 0u;
+  sel &= nw >= 32 ? ~0u : (nw <= 0 ? 0u : (1u << nw) - 1u);
+  int total, unused;
+  const int2 r = block_exclusive_scan2(__builtin_popcount(sel), 0, sh.scan, &total, &unused);
+  if (tid < KEYS / 32) {
+    bits32[tid] = sel;
+    ((int *)sh.eqbits)[tid] = r.x;
+  }
+  __syncthreads();
+  return total;
+}
+
+template <int EPT>
+__global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_chunk_kernel(IndexerParams p) {
+  constexpr int KEYS = EPT * kTopkThreads;
+  __shared__ __attribute__((aligned(16))) TopkShared<KEYS> sh;
+  const int t = blockIdx.y, c0 = blockIdx.x * p.chunk;
+  const int tid = threadIdx.x;
+  float *chunk = p.scores + (int64_t)t * p.S + c0;
+  const RowCodes rc = load_row_codes(p, t);
+  uint32_t key[EPT];
+  load_keys(chunk, min(p.chunk, p.S - c0), key);
+  const int n_row = candidates(p, t), n = min(n_row - c0, p.chunk);
+  if (n_row <= p.topk) return;  // the row takes all its candidates
+  if (n <= p.topk) {            // few or none: all are listed
+    to_keys(max(n, 0), key);
+    __syncthreads();  // every wave's keys have arrived: the list may take their place
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+      const int i = e * kTopkThreads + tid;
+      if (i < p.list_len) {
+        ((uint32_t *)chunk)[i] = i < n ? max(key[e], 1u) : 0u;
+        ((int32_t *)chunk)[p.list_len + i] = c0 + i;
+      }
+    }
+    return;
+  }
+  clear_counts(sh);
+  bound_shares(p, sh, rc, c0 >> 4, (c0 + n + 15) >> 4);
+  __syncthreads();
+  bound(sh);
+  to_keys(n, key);
+  uint32_t prefix, mask;
+  int need;
+  find_bin(p, sh, key, KEYS - n, prefix, mask, need);
+  const float band = sh.band;
+  const uint32_t lo = max(order_key(key_value(prefix) - band), 1u);
+  mark_taken(sh, n, key, ~0u, lo - 1, ~0u);  // every key from lo on
+  store_row_pieces(p, sh, rc);
+  __syncthreads();
+  int total = rank_marks<KEYS>(sh, n);
+  if (!(band == band && total <= p.list_len)) {  // uniform
+    if (!(band == 0.f)) {
+      exact_scores(p, sh, (n + 15) >> 4, [&](int b, int c) { return min(c0 + b * 16 + c, p.S - 1); },
+                   [&](int b, int c, float v) {
+                     if (b * 16 + c < n) chunk[b * 16 + c] = v;
+                   });
+      load_keys(chunk, n, key);
+      to_keys(n, key);
+    }
+    mark_exact(p, sh, n, key, KEYS - n);
+    total = rank_marks<KEYS>(sh, n);
+  }
+  write_list(p, sh, n, c0, key, total, chunk);
+}
+
+// Selection of a row from its chunks' lists (EPT * 1024 places, list_len per list).
+template <int EPT>
+__global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_merge_kernel(IndexerParams p) {
+  constexpr int KEYS = EPT * kTopkThreads;
+  __shared__ __attribute__((aligned(16))) TopkShared<KEYS> sh;
+  const int t = blockIdx.x;
+  const int tid = threadIdx.x;
+  float *row = p.scores + (int64_t)t * p.S;
+  int32_t *out = p.out + (int64_t)t * p.topk;
+  const RowCodes rc = load_row_codes(p, t);
+  // place i: entry i % list_len (a power of two, at least 1024) of list i / list_len
+  auto entry = [&](int i) { return (i >> p.list_shift) * p.chunk + (i & (p.list_len - 1)); };
+  const int places = p.n_chunks << p.list_shift;
+  uint32_t key[EPT];
+  auto load_lists = [&]() {
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(row, 0, p.S * 4, kBufferFlags);
+#pragma unroll
+    for (int e = 0; e < EPT; ++e)
+      key[e] = e * kTopkThreads < places
+                   ? __builtin_amdgcn_raw_buffer_load_b32(rs, tid * 4, entry(e * kTopkThreads) * 4, 0)
+                   : 0u;
+  };
+  load_lists();
+  const int n = candidates(p, t);
+  if (take_all(p, t, out, n)) return;  // (nothing was listed)
+
+  auto position = [&](int i) { return ((const int32_t *)row)[entry(i) + p.list_len]; };
+  clear_counts(sh);
+  bound_shares(p, sh, rc, 0, (n + 15) >> 4);
+  __syncthreads();
+  bound(sh);
+  uint32_t prefix, mask;
+  int need;
+  find_bin(p, sh, key, 0, prefix, mask, need);  // (empty entries are the lowest keys)
+  const float band = sh.band;
+  mark_taken(sh, KEYS, key, max(order_key(key_value(prefix) - band), 1u),
+             order_key(key_value(prefix | 0xffffu) + band), prefix | 0xffffu);
+  store_row_pieces(p, sh, rc);
+  __syncthreads();
+  const int n_open = sh.n_cand;
+  if (band == band && n_open <= kMaxOpen) {  // uniform
+    exact_scores(p, sh, (n_open + 15) >> 4,
+                 [&](int b, int c) { return position((int)sh.cand[min(b * 16 + c, n_open - 1)].y); },
+                 [&](int b, int c, float v) {
+                   if (b * 16 + c < n_open) sh.cand[b * 16 + c].x = max(order_key(v), 1u);
+                 });
+    rank_open(sh, n_open, need + sh.n_above);
+    write_marked<KEYS>(p, sh, t, KEYS, out, position);
+    return;
+  }
+  // every listed position's exact score, then the selection from those
+  if (!(band == 0.f)) {
+    uint32_t *keys = (uint32_t *)row;
+    exact_scores(p, sh, places >> 4,
+                 [&](int b, int c) { return keys[entry(b * 16 + c)] != 0 ? position(b * 16 + c) : 0; },
+                 [&](int b, int c, float v) {
+                   uint32_t *k = keys + entry(b * 16 + c);
+                   if (*k != 0) *k = max(order_key(v), 1u);
+                 });
+    load_lists();
+  }
+  mark_exact(p, sh, KEYS, key, 0);
+  write_marked<KEYS>(p, sh, t, KEYS, out, position);
 }
 
 // Rows longer than the register kernel holds: the same selection, reading
@@ -1079,7 +1316,29 @@ hipError_t launch_estimate(const IndexerParams &p, dim3 grid, hipStream_t stream
 
 }  // namespace
 
-bool estimates_apply(const IndexerParams &p) { return p.S <= kTopkThreads * kMaxRegEpt; }
+// Rows longer than 32768 positions run in chunks of at most that: as few as
+// possible (the lists of all must fit one workgroup's registers, and two
+// list lengths a chunk).  A list holds twice the top-k or so: the chunk's k
+// largest, and those whose estimates are too close to tell.
+static bool chunk_plan(const IndexerParams &p, int *chunk, int *n_chunks, int *list_shift) {
+  constexpr int kMax = kTopkThreads * kMaxRegEpt;
+  const int c = (p.S + kMax - 1) / kMax;
+  const int len = ((p.S + c - 1) / c + 15) / 16 * 16;
+  int shift = 10;
+  while ((1 << shift) < p.topk + 512) {
+    if (++shift > 15) return false;
+  }
+  if ((int64_t)c << shift > kMax || p.S - (int64_t)(c - 1) * len < 2 << shift) return false;
+  *chunk = len;
+  *n_chunks = c;
+  *list_shift = shift;
+  return true;
+}
+
+bool estimates_apply(const IndexerParams &p) {
+  int chunk, n, shift;
+  return p.T <= 65535 && (p.S <= kTopkThreads * kMaxRegEpt || chunk_plan(p, &chunk, &n, &shift));
+}
 
 // Few tokens: the estimate kernel is bound by latency and prepares K on its way
 // (a launch less: 3 tokens, 2500 positions, 32 heads 20.6 -> 16.1 us); from 9
@@ -1116,10 +1375,26 @@ hipError_t launch_estimates(const IndexerParams &pin, hipStream_t stream) {
   }
 }
 
+static hipError_t launch_topk_chunks(const IndexerParams &pin, hipStream_t stream) {
+  IndexerParams p = pin;
+  if (!chunk_plan(p, &p.chunk, &p.n_chunks, &p.list_shift)) return hipErrorInvalidValue;
+  p.list_len = 1 << p.list_shift;
+  const dim3 block(kTopkThreads), grid(p.n_chunks, p.T);
+  hipLaunchKernelGGL(dsa_idx_topk_chunk_kernel<kMaxRegEpt>, grid, block, 0, stream, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const int places = p.n_chunks << p.list_shift;
+  if (places <= kTopkThreads * 8) hipLaunchKernelGGL(dsa_idx_topk_merge_kernel<8>, dim3(p.T), block, 0, stream, p);
+  else if (places <= kTopkThreads * 16) hipLaunchKernelGGL(dsa_idx_topk_merge_kernel<16>, dim3(p.T), block, 0, stream, p);
+  else hipLaunchKernelGGL(dsa_idx_topk_merge_kernel<kMaxRegEpt>, dim3(p.T), block, 0, stream, p);
+  return hipGetLastError();
+}
+
 hipError_t launch_topk(const IndexerParams &p, hipStream_t stream) {
   if (p.S <= kTopkThreads * 8) return launch_topk_regs<8>(p, stream);
   if (p.S <= kTopkThreads * 16) return launch_topk_regs<16>(p, stream);
   if (p.S <= kTopkThreads * kMaxRegEpt) return launch_topk_regs<kMaxRegEpt>(p, stream);
+  if (p.estimated) return launch_topk_chunks(p, stream);
   hipLaunchKernelGGL(dsa_idx_topk_stream_kernel, dim3(p.T), dim3(kTopkThreads), 0, stream, p);
   return hipGetLastError();
 }

@@ -566,7 +566,12 @@ def _full_range(d, g):
 # and to the row length, token counts around the pairs and fours of the waves
 @pytest.mark.parametrize("T,Hi,S,topk", [(1, 64, 65, 64), (2, 16, 8192, 2048), (3, 32, 8193, 1), (5, 48, 16384, 2048),
                                          (7, 64, 16385, 16000), (9, 64, 32768, 2048), (6, 16, 32751, 2047),
-                                         (33, 64, 2049, 2048)])
+                                         (33, 64, 2049, 2048),
+                                         # chunks and their lists: the shortest row, chunk ends inside a
+                                         # block, 2 to 9 lists of 1024 to 4096 places, top-k above them
+                                         (2, 64, 32769, 2048), (9, 32, 40007, 700), (3, 64, 131071, 2048),
+                                         (2, 16, 262144, 2048), (2, 16, 262145, 512), (3, 16, 70000, 3584),
+                                         (2, 16, 50000, 9000)])
 @pytest.mark.parametrize("full_range", [False, True])
 def test_selection_without_scores_matches_oracle(T, Hi, S, topk, full_range):
     gen = torch.Generator().manual_seed(S + T)
@@ -609,6 +614,9 @@ def _hard(kind, T, Hi, S):
         k *= torch.exp2(torch.randint(-9, 9, (S, 128), generator=gen).float())
     elif kind == "zero weights":
         d["weights"][::2] = 0.0
+    elif kind == "zero queries":
+        d["q_idx"] = d["q_idx"].clone()
+        d["q_idx"][1::2] = 0
     elif kind == "tiny weights":
         d["weights"] *= 1e-30
         d["weights"][0] *= 1e-12          # subnormal products
@@ -630,9 +638,9 @@ def _hard(kind, T, Hi, S):
     return d
 
 
-@pytest.mark.parametrize("S", [6000, 20000])
+@pytest.mark.parametrize("S", [6000, 20000, 40000])
 @pytest.mark.parametrize("kind", ["many equal rows", "nearly equal rows", "outlier rows", "outlier scales", "zero rows",
-                                  "wide exponents", "zero weights", "tiny weights", "huge weights",
+                                  "wide exponents", "zero weights", "zero queries", "tiny weights", "huge weights",
                                   "weights not finite", "scales not finite", "NaN codes"])
 def test_selection_without_scores_of_hard_rows(kind, S):
     """Rows whose estimates leave many positions open or whose error bound is
@@ -646,12 +654,13 @@ def test_selection_without_scores_of_hard_rows(kind, S):
 
 
 def test_selection_without_scores_after_nan_filled_lds():
-    d = _full_range(workloads.indexer_inputs(T=5, Hi=64, S=20000, seed=77), torch.Generator().manual_seed(78))
-    ref, _ = _oracle(d, 2048)
-    g = workloads.to_device(d, DEV)
-    for r in range(3):
-        fill_lds_with_nan(DEV)
-        print(f"NaN-filled LDS selection call {r}", flush=True)
-        out = run_indexer_and_topk(g["q_idx"], g["k_idx"], g["k_scale"], g["weights"], g["causal_limit"], 2048)
-        torch.cuda.synchronize()
-        assert np.array_equal(np.sort(out.cpu().numpy(), axis=1), np.sort(ref, axis=1))
+    for S in (20000, 45000):
+        d = _full_range(workloads.indexer_inputs(T=5, Hi=64, S=S, seed=77), torch.Generator().manual_seed(78))
+        ref, _ = _oracle(d, 2048)
+        g = workloads.to_device(d, DEV)
+        for r in range(3):
+            fill_lds_with_nan(DEV)
+            print(f"NaN-filled LDS selection S={S} call {r}", flush=True)
+            out = run_indexer_and_topk(g["q_idx"], g["k_idx"], g["k_scale"], g["weights"], g["causal_limit"], 2048)
+            torch.cuda.synchronize()
+            assert np.array_equal(np.sort(out.cpu().numpy(), axis=1), np.sort(ref, axis=1))
