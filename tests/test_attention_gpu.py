@@ -665,3 +665,28 @@ def test_captured_counters_outlive_a_larger_eager_call():
         assert torch.equal(gout, ref_out) and torch.equal(glse, ref_lse), f"replay {i}"
         assert int((cap != 0).sum()) == 0
     assert all(bool((f == -1).all()) for f in filler)
+
+
+# Every layout: four-wave kernel sorted (one chunk) and unsorted (splits), ring
+# kernels of 2 x 4 slices, 4 and 8 head groups.  Valid counts around the 16-key
+# blocks, the 32-key tiles, the four waves' quarters and the slot-id ring.
+@pytest.mark.parametrize("H,T,splits", [(16, 44, 1), (16, 44, 4), (16, 44, 0), (32, 132, 1), (64, 66, 1),
+                                        (128, 132, 1), (128, 22, 0)])
+def test_rows_padded_at_their_end(H, T, splits):
+    counts = [0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 129, 511, 512, 513, 1023, 1024, 1025, 1535, 2047, 2048]
+    K, slots = 2048, 4096
+    g = torch.Generator().manual_seed(H * 100 + T + splits)
+    d = workloads.attention_inputs(T, H, K, slots // 64, 64, H + T)
+    d.pop("gen")
+    idx = torch.full((T, K), -1, dtype=torch.int32)
+    for t in range(T):
+        n = counts[t % len(counts)]
+        idx[t, :n] = torch.randperm(slots, generator=g)[:n].sort().values.to(torch.int32)
+        if (t // len(counts)) % 2 == 1:  # padding inside the row as well
+            idx[t, :n][torch.rand(n, generator=g) < 0.3] = -1
+    d.update(sparse_indices=idx, sm_scale=workloads.SM_SCALE)
+    print(f"padded rows H={H} T={T} splits={splits}", flush=True)
+    out, lse = _run(kernel_splitk, d, SPLIT_K=splits) if splits else _run(kernel, d)
+    _assert_parity(out, lse, *_oracle(d), f"padded rows H={H} splits={splits}")
+    empty = [t for t in range(T) if bool((idx[t] < 0).all())]
+    assert empty and torch.isneginf(lse[empty]).all() and (out[empty] == 0).all()
