@@ -75,10 +75,13 @@
 // feature f0+i of keys 0..3: one half of an A operand of V^T.
 #include "dsa_internal.h"
 
+#include <type_traits>
+
 namespace dsa {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -334,6 +337,10 @@ __device__ __forceinline__ void for_tr_batches(const char *vsrc, Fn &&fn) {
   }
 }
 
+__device__ __forceinline__ uint32_t lds_u32(const char *p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p;
+}
+
 // Workgroup barrier for LDS data only: this wave's LDS accesses complete
 // (lgkmcnt(0)), then s_barrier, in one statement the compiler moves no memory
 // access across.  Unlike __syncthreads() it leaves vector-memory loads (and
@@ -420,7 +427,7 @@ __device__ __forceinline__ f32x4 qk_part(int part, const char *rowp, const char 
   return kChains == 2 ? c[0] + c[1] : c[0];
 }
 
-// Fused QK/PV loop (one-slice layouts, one head group per wave): S^T of
+// Fused QK/PV loop (eight waves, one head group per wave): S^T of
 // both 16-key blocks of tile i interleaved with the PV product of tile i-1.
 // Step K (0..35) is QK k-step K % 18 of key block K / 18 and, for K < 32,
 // feature block K of the PV product (its V^T halves of key block 0 and 1).
@@ -499,12 +506,201 @@ __device__ __forceinline__ void qk_pv_tile(const FusedAddr &a, const QkOperands<
   qk_pv_steps(a, q, p_hi, p_lo, acc, s, kq, vt);
 }
 
+// ---- four-wave one-slice layout: the tile as one stream of LDS reads and MFMAs.
+// One wave per SIMD has nothing but its own instructions to hide latency
+// with, so everything a tile needs is one straight line.  Items 0..17 are the
+// QK k-steps of tile i (K operands of both 16-key blocks), items 18..49 the
+// 16-feature blocks of tile i-1's PV product (V^T of both key blocks), with
+// the softmax of tile i between their MFMAs.  Every item is two LDS reads,
+// issued kAhead items before its MFMAs, so waiting for an item is one exact
+// lgkmcnt count (1, 2 and 3 ahead: 106, 103 and 105 us for 300 tokens of 64
+// heads at top-k 1024).
+constexpr int kQkItems = 18;
+constexpr int kItems = kQkItems + 32;
+constexpr int kAhead = 2;
+// Softmax steps (softmax_step in the kernel), one after each PV MFMA from the
+// one after the scores are settled.
+constexpr int kSettle = 4;
+constexpr int kSoftmaxSteps = 5 + 4 * 7;
+static_assert(kSettle + kSoftmaxSteps <= 64, "one step after each PV MFMA");
+
+// LDS addresses of this lane's QK operand rows of key block 0 (ckv row; kpe
+// row + 128 g) and of its V^T reads (as in the pv stage).  Key block 1 lies
+// at constant offsets: the next ckv row (ring_row), two kpe groups on.
+struct TileAddr {
+  uint32_t q, k, v;
+};
+
+// Operand registers of the items in flight, one set per item modulo kAhead + 1.
+struct ItemRegs {
+  u32x4 k[kAhead + 1][2];
+  u32x2 v[kAhead + 1][2];
+};
+
+template <int I>
+__device__ __forceinline__ void item_issue(const TileAddr &a, ItemRegs &r) {
+  constexpr int kSet = I % (kAhead + 1);
+  if constexpr (I < kQkItems) {
+    constexpr int kOff = I < 16 ? I * 64 : (I - 16) * 512;
+    asm volatile(
+        "ds_read_b128 %0, %2 offset:%3\n\t"
+        "ds_read_b128 %1, %2 offset:%4"
+        : "=&v"(r.k[kSet][0]), "=&v"(r.k[kSet][1])
+        : "v"(I < 16 ? a.q : a.k), "i"(kOff), "i"(kOff + (I < 16 ? kCkvPitch : 2 * kKpeGroupPitch))
+        : "memory");
+  } else {
+    constexpr int kOff = (I - kQkItems) * 32;
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %2 offset:%3\n\t"
+        "ds_read_b64_tr_b16 %1, %2 offset:%4"
+        : "=&v"(r.v[kSet][0]), "=&v"(r.v[kSet][1])
+        : "v"(a.v), "i"(kOff), "i"(kCkvPitch + kOff)
+        : "memory");
+  }
+}
+
+// Both of the next two wait until at most N LDS operations issued after the
+// item's reads are outstanding (LDS operations complete in issue order; any
+// other operation counted meanwhile only makes the wait longer).
+//
+// S^T += K Q^T of a k-step (FIRST: starts from zero).  The MFMAs of this
+// stream are written out: left to itself the compiler places the result of
+// each where it likes and copies accumulators between registers (64 heads,
+// 300 tokens, top-k 2048: 213 us with builtins, 185 so).  scores_settled and
+// accumulators_settled stand for the hazards it then does not know of.
+template <int N, bool FIRST>
+__device__ __forceinline__ void item_qk(const u32x4 (&k)[2], const bf16x8 &q, f32x4 (&s)[2]) {
+  if constexpr (FIRST)
+    asm volatile(
+        "s_waitcnt lgkmcnt(%5)\n\t"
+        "v_mfma_f32_16x16x32_bf16 %0, %2, %4, 0\n\t"
+        "v_mfma_f32_16x16x32_bf16 %1, %3, %4, 0"
+        : "=&v"(s[0]), "=&v"(s[1])
+        : "v"(k[0]), "v"(k[1]), "v"(q), "n"(N)
+        : "memory");
+  else
+    asm volatile(
+        "s_waitcnt lgkmcnt(%5)\n\t"
+        "v_mfma_f32_16x16x32_bf16 %0, %2, %4, %0\n\t"
+        "v_mfma_f32_16x16x32_bf16 %1, %3, %4, %1"
+        : "+&v"(s[0]), "+&v"(s[1])
+        : "v"(k[0]), "v"(k[1]), "v"(q), "n"(N)
+        : "memory");
+}
+// The V^T registers are in/out operands, so their uses cannot move above the wait.
+template <int N>
+__device__ __forceinline__ void item_wait(u32x2 (&v)[2]) {
+  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(v[0]), "+v"(v[1]) : "n"(N) : "memory");
+}
+// O^T += V^T P^T of one feature block, in place.
+__device__ __forceinline__ void pv_mfma(f32x4 &acc, const bf16x8 &av, const u32x4 &p) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(av), "v"(p));
+}
+// At least STATES wait states between item_qk's last MFMA and the first read
+// of its result (16 are more than an MFMA of this shape asks for; in the
+// stream kSettle + 1 PV MFMAs, four states each, stand in between as well).
+template <int STATES>
+__device__ __forceinline__ void scores_settled(f32x4 (&s)[2]) {
+  asm volatile("s_nop %2" : "+v"(s[0]), "+v"(s[1]) : "n"(STATES - 1));
+}
+// The same between the last pv_mfma and other uses of the accumulators.
+template <int N>
+__device__ __forceinline__ void accumulators_settled(f32x4 (&acc)[N]) {
+  asm volatile("s_nop 15");
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+a"(acc[i]));
+}
+
+struct TileState {
+  f32x4 s[2];         // S^T of tile i, per key block
+  u32x4 p_hi, p_lo;   // probabilities of tile i-1 (8 bf16 each)
+};
+
+// Items FROM .. TO - 1; side(item) after each QK item, gap(m) after PV MFMA m.
+template <int I, int FROM, int TO, typename Side, typename Gap>
+__device__ __forceinline__ void run_items(const TileAddr &a, const QkOperands<1> &q, f32x4 (&acc)[32], TileState &st,
+                                          ItemRegs &r, const bf16x8 &av1, Side &&side, Gap &&gap) {
+  if constexpr (I < TO) {
+    static_assert(kAhead == 2 && TO - FROM > 2, "items issued before the first");
+    if constexpr (I == FROM) {
+      item_issue<I>(a, r);
+      item_issue<I + 1>(a, r);
+    }
+    if constexpr (I + kAhead < TO) item_issue<I + kAhead>(a, r);
+    constexpr int kBehind = TO - 1 - I < kAhead ? TO - 1 - I : kAhead;
+    constexpr int kSet = I % (kAhead + 1);
+    if constexpr (I < kQkItems) {
+      item_qk<2 * kBehind, I == 0>(r.k[kSet], I < 16 ? q.nope[I] : q.pe32[I - 16], st.s);
+      side(std::integral_constant<int, I>{});
+      run_items<I + 1, FROM, TO>(a, q, acc, st, r, av1, side, gap);
+    } else {
+      constexpr int K = I - kQkItems;
+      item_wait<2 * kBehind>(r.v[kSet]);
+      const bf16x8 av = __builtin_bit_cast(
+          bf16x8, u32x4{r.v[kSet][0][0], r.v[kSet][0][1], r.v[kSet][1][0], r.v[kSet][1][1]});
+      // a block's second product follows the next block's first: no two MFMAs
+      // in a row on one accumulator
+      pv_mfma(acc[K], av, st.p_hi);
+      gap(std::integral_constant<int, 2 * K>{});
+      if constexpr (K > 0) pv_mfma(acc[K - 1], av1, st.p_lo);
+      gap(std::integral_constant<int, 2 * K + 1>{});
+      if constexpr (K == 31) pv_mfma(acc[K], av, st.p_lo);
+      run_items<I + 1, FROM, TO>(a, q, acc, st, r, av, side, gap);
+    }
+  }
+}
+
+template <int FROM, int TO, typename Side, typename Gap>
+__device__ __forceinline__ void tile_items(const TileAddr &a, const QkOperands<1> &q, f32x4 (&acc)[32], TileState &st,
+                                           Side &&side, Gap &&gap) {
+  ItemRegs r;
+  run_items<FROM, FROM, TO>(a, q, acc, st, r, bf16x8{}, side, gap);
+}
+
+// The rare rescaling of O^T accumulators that live in AGPRs.  The empty asm
+// statements pin them there around it: left to itself the compiler copies all
+// of them to VGPRs at the head of every loop iteration, ready for this branch
+// -- in the wave kernel 128 moves per 16-key block, and the registers they
+// take push Q^T into AGPRs, which costs four more moves before most QK MFMAs
+// (2048 prefill tokens of 16 heads 417 -> 350 us, 300 tokens 104 -> 84).
+template <int N>
+__device__ __forceinline__ void rescale(f32x4 (&acc)[N], float alpha) {
+  asm volatile("s_nop 15");
+#pragma unroll
+  for (int i = 0; i < N; ++i) {  // one at a time: few VGPRs for a rare step
+    asm volatile("" : "+a"(acc[i]));
+    acc[i] *= alpha;
+    asm volatile("" : "+a"(acc[i]));
+  }
+}
+
+// fn(std::integral_constant<int, I>{}) for I = 0 .. N - 1.
+template <int N, int I = 0, typename Fn>
+__device__ __forceinline__ void for_each_int(Fn &&fn) {
+  if constexpr (I < N) {
+    fn(std::integral_constant<int, I>{});
+    for_each_int<N, I + 1>(fn);
+  }
+}
+
+// Max over the four lanes that hold one head (lane groups g = 0..3).
+__device__ __forceinline__ float max_lane_groups(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  const float x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// Where this lane's key of a tile is gathered from.
+struct KeySrc {
+  uint32_t co, ko;    // narrow: byte offsets of its ckv row and of this lane's 16-byte kpe chunk
+  uint64_t ckv, kpe;  // otherwise: row addresses
+};
 // Source of one wave's share of a tile gather (see tile_src in the kernel).
 template <int ROWS>
 struct GatherSrc {
   uint32_t row[ROWS];  // narrow: ckv byte offset of each row this wave gathers
-  uint32_t ko;         // narrow: kpe byte offset of this lane's 16-byte chunk
-  uint64_t ckv, kpe;   // otherwise: row addresses of this lane's key
+  KeySrc key;
 };
 
 // W waves per workgroup; FS waves share one 16-head group, each owning
@@ -742,11 +938,11 @@ __global__ __launch_bounds__(W * 64, 1) void dsa_attn_ring_kernel(AttnParams p) 
     if (lane == 0) *last_of_wave(wave) = last;
   }
 
-  // The fused QK/PV loop of the one-slice layouts runs a PV step on the
+  // The fused QK/PV loop of the eight-wave layout runs a PV step on the
   // first tile too, from the stage of tile -1 with zero probabilities: that
   // stage's ckv rows are zeroed here (its first gather is issued after the
   // first tile is computed), so the step adds exact zeros.
-  if constexpr (FS == 1) {
+  if constexpr (FS == 1 && W == 8) {
     u32x4 *z = (u32x4 *)(lds + (kStages - 1) * kStageBytes);
     for (int i = threadIdx.x; i < kCkvStageBytes / 16; i += W * 64) z[i] = u32x4{0u, 0u, 0u, 0u};
   }
@@ -788,26 +984,31 @@ __global__ __launch_bounds__(W * 64, 1) void dsa_attn_ring_kernel(AttnParams p) 
   // frees the stage, off the path between the barriers); fire_tile issues the
   // DMAs into stage j % kStages.
   using TileSrc = GatherSrc<R::kRows>;
-  auto tile_src = [&](int j) {
-    TileSrc a;
-    const int32_t *ids = slots + (j % L::kRingTiles) * kKeysPerTile;  // refilled ids are raw
-    note_refilled_mask(j, ids);
+  auto key_src = [&](int sl) {
+    KeySrc a;
+    const bool ok = (uint32_t)sl < (uint32_t)p.num_slots;  // -1 wraps to 2^32 - 1
     if constexpr (NARROW) {
-      const uint32_t sl = (uint32_t)ids[grp * 8 + (lane & 7)];
-      const bool ok = sl < (uint32_t)p.num_slots;  // -1 wraps to 2^32 - 1
-      const uint32_t co = ok ? __umul24(sl, p.ckv_rs) : kOOB;
-#pragma unroll
-      for (int m = 0; m < R::kRows; ++m) a.row[m] = __builtin_amdgcn_readlane(co, row0 + m);
-      a.ko = (ok ? __umul24(sl, p.kpe_rs) : kOOB) + (lane >> 3) * 16;
+      a.co = ok ? __umul24((uint32_t)sl, p.ckv_rs) : kOOB;
+      a.ko = (ok ? __umul24((uint32_t)sl, p.kpe_rs) : kOOB) + (lane >> 3) * 16;
     } else {
-      const int sl = ids[grp * 8 + (lane & 7)];
       a.ckv = a.kpe = (uint64_t)(const char *)g_zero_row;
-      if (sl >= 0 && (int64_t)sl < p.num_slots) {
+      if (ok) {
         const uint32_t pg = (uint32_t)(((uint64_t)(uint32_t)sl * p.ps_magic) >> (31 + p.ps_shift));
         const uint32_t of = (uint32_t)sl - pg * (uint32_t)p.page_size;
         a.ckv = (uint64_t)(p.ckv + (int64_t)pg * p.ckv_sp + (int64_t)of * p.ckv_so);
         a.kpe = (uint64_t)(p.kpe + (int64_t)pg * p.kpe_sp + (int64_t)of * p.kpe_so);
       }
+    }
+    return a;
+  };
+  auto tile_src = [&](int j) {
+    TileSrc a;
+    const int32_t *ids = slots + (j % L::kRingTiles) * kKeysPerTile;  // refilled ids are raw
+    note_refilled_mask(j, ids);
+    a.key = key_src(ids[grp * 8 + (lane & 7)]);
+    if constexpr (NARROW) {
+#pragma unroll
+      for (int m = 0; m < R::kRows; ++m) a.row[m] = __builtin_amdgcn_readlane(a.key.co, row0 + m);
     }
     return a;
   };
@@ -818,14 +1019,14 @@ __global__ __launch_bounds__(W * 64, 1) void dsa_attn_ring_kernel(AttnParams p) 
 #pragma unroll
       for (int m = 0; m < R::kRows; ++m)
         lds_dma16_buf(ckv_rsrc, st + ring_row(grp * 8 + row0 + m) * kCkvPitch, a.row[m] + lane * 16);
-      if (kpe_lane) lds_dma16_buf(kpe_rsrc, kdst, a.ko);
+      if (kpe_lane) lds_dma16_buf(kpe_rsrc, kdst, a.key.ko);
     } else {
 #pragma unroll
       for (int m = 0; m < R::kRows; ++m) {
-        const char *src = (const char *)readlane64(a.ckv, row0 + m) + lane * 16;
+        const char *src = (const char *)readlane64(a.key.ckv, row0 + m) + lane * 16;
         lds_dma16(src, st + ring_row(grp * 8 + row0 + m) * kCkvPitch);
       }
-      if (kpe_lane) lds_dma16((const char *)a.kpe + (lane >> 3) * 16, kdst);
+      if (kpe_lane) lds_dma16((const char *)a.key.kpe + (lane >> 3) * 16, kdst);
     }
   };
 
@@ -944,7 +1145,10 @@ __global__ __launch_bounds__(W * 64, 1) void dsa_attn_ring_kernel(AttnParams p) 
   // two teams of waves (W == 8, one-slice): waves 0-3 and 4-7, one of each
   // per SIMD, half an iteration apart (below); they keep two tiles ahead
   constexpr bool kTeams = FS == 1 && W == 8;
-  const int pre = min(n_tiles, kTeams ? 2 : kStages - 1);
+  // one line per tile (W == 4, one-slice; see item_issue): two tiles ahead,
+  // past the last one zero rows
+  constexpr bool kStream = FS == 1 && W == 4;
+  const int pre = kStream ? 2 : min(n_tiles, kTeams ? 2 : kStages - 1);
   for (int j = 0; j < pre; ++j) fire_tile(j, tile_src(j));
 
   // the first ring pass's tile masks, built while the first tiles are in flight
@@ -974,134 +1178,279 @@ __global__ __launch_bounds__(W * 64, 1) void dsa_attn_ring_kernel(AttnParams p) 
   // stage then receives tile i+3.  Tile i-1 stays in LDS one iteration
   // longer, which is what the fourth stage is for; two tiles remain in
   // flight.
-  bf16x8 p_hi = {}, p_lo = {};
-  auto lds_addr = [](const char *q) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)q;
-  };
-  const int k0 = key_of_row(r16), k1 = 16 + key_of_row(r16);
-  if constexpr (kTeams) {
-    const bool team_b = wave >= 4;
-    f32x4 sb[2];  // S^T of the wave's current tile, from its QK/PV step to its softmax
-    auto fused = [&](int i, f32x4 (&sacc)[2]) {
-      const char *st_ckv = lds + (i & (kStages - 1)) * kStageBytes;
-      const char *st_prev = lds + ((i + kStages - 1) & (kStages - 1)) * kStageBytes;
-      const char *st_kpe = st_ckv + kCkvStageBytes;
-      const FusedAddr fa = {
-          lds_addr(st_ckv + ring_row(k0) * kCkvPitch + g * 16), lds_addr(st_ckv + ring_row(k1) * kCkvPitch + g * 16),
-          lds_addr(st_kpe + kpe_group_off(k0 >> 3) + (k0 & 7) * 16 + g * 128),
-          lds_addr(st_kpe + kpe_group_off(k1 >> 3) + (k1 & 7) * 16 + g * 128),
-          lds_addr(st_prev + ring_row(kbase + 2 * (r16 >> 2)) * kCkvPitch + 4 * (r16 & 3) * 2)};
-      qk_pv_tile(fa, qreg, p_hi, p_lo, acc, sacc);
-    };
-    // Both teams run the same loop (X_j, fused j, Y_j, softmax j); team B
-    // passes one extra barrier first and team A one after, so the barriers
-    // pair A's X_j with B's Y_{j-1} and A's Y_j with B's X_j: each team's
-    // QK/PV of a tile runs while the other team does its softmax.  Before a
-    // barrier that lets either team compute tile j, both teams' shares of
-    // tile j have landed: A waits before X_j, B before Y_{j-1}.  The stage of
-    // tile j-2 is free once both teams passed their fused step j-1, i.e.
-    // after the pair (A's X_j, B's Y_{j-1}): B fires its share of tile j+2
-    // right after that pair (before its softmax of tile j-1), A after its
-    // softmax of tile j (while B runs its fused step j).
-    int fired = pre - 1;  // last tile whose share this wave has issued
-    auto wait_own = [&](int j) {  // this wave's share of tile j landed
-      const int ahead = fired - j;
-      if (ahead >= 2)
-        wait_vmcnt<2 * R::kLoads>();
-      else if (ahead == 1)
-        wait_vmcnt<R::kLoads>();
-      else
-        wait_vmcnt<0>();
-    };
-    if (team_b) {
-      // this barrier is team A's X_0: team B's share of tile 0 lands first
-      wait_own(0);
+  if constexpr (kStream) {
+    if (n_tiles > 0) {
+      // Iteration i runs QK of tile i, then the PV product of tile i-1 with
+      // the softmax of tile i between its MFMAs.  One barrier a tile: past it
+      // every wave's share of tile i has landed and every wave is done with
+      // tile i-2, whose stage takes tile i+2 (issued between the QK MFMAs;
+      // past the last tile zero rows, so every wait is one count).  The
+      // softmax of a tile as a block of its own, after a fused QK/PV loop and
+      // with a second barrier, left the matrix cores idle for it: H=64,
+      // top-k 2048, T=64 50 -> 44 us, T=300 225 -> 185; H=128, T=32 48 -> 43.
+      const int k0 = key_of_row(r16);
+      const uint32_t base = lds_u32(lds);
+      const uint32_t q0 = base + ring_row(k0) * kCkvPitch + g * 16;
+      const uint32_t kp0 = base + kCkvStageBytes + kpe_group_off(k0 >> 3) + (k0 & 7) * 16 + g * 128;
+      const uint32_t v0 = base + ring_row(kbase + 2 * (r16 >> 2)) * kCkvPitch + 4 * (r16 & 3) * 2;
+      const uint32_t id0 = base + kStages * kStageBytes + (grp * 8 + (lane & 7)) * 4;
+      auto addr = [&](int i) {
+        const uint32_t cur = (i & (kStages - 1)) * kStageBytes;
+        const uint32_t prev = ((i + kStages - 1) & (kStages - 1)) * kStageBytes;
+        return TileAddr{q0 + cur, kp0 + cur, v0 + prev};
+      };
+      int id = slots[2 * kKeysPerTile + grp * 8 + (lane & 7)];  // slot id of this lane's key of the tile issued next
+      KeySrc src = key_src(id);
+      auto piece = [&](int j, auto M) {  // one DMA of tile j's gather
+        constexpr int m = decltype(M)::value;
+        char *st = lds + (j & (kStages - 1)) * kStageBytes;
+        if constexpr (m < R::kRows) {
+          char *dst = st + ring_row(grp * 8 + m) * kCkvPitch;
+          if constexpr (NARROW)
+            lds_dma16_buf(ckv_rsrc, dst, (uint32_t)__builtin_amdgcn_readlane(src.co, m) + lane * 16);
+          else
+            lds_dma16((const char *)readlane64(src.ckv, m) + lane * 16, dst);
+        } else {
+          char *dst = st + kCkvStageBytes + kpe_group_off(grp);
+          if constexpr (NARROW)
+            lds_dma16_buf(kpe_rsrc, dst, src.ko);
+          else
+            lds_dma16((const char *)src.kpe + (lane >> 3) * 16, dst);
+        }
+      };
+      TileState st;
+      float alpha = 1.f, d[8], x[2], psum = 0.f;
+      bool moved = false;
+      u32x4 n_hi, n_lo;
+      uint32_t vmask = 0;
+      const float c = p.scale_log2;
+      // ---- online softmax of tile i, cut into steps of one to three
+      // instructions that go between the PV MFMAs, where a wave can issue
+      // about that many before the next one is due.  This lane: head r16 of
+      // each group; element 4 b + k holds key b*16 + kbase + 2k.  The
+      // reference m_run only moves when some score overshoots it by more than
+      // kRescaleSlack (always on the first valid tile, where m_run = -inf);
+      // the accumulators, which then hold tiles before i only, are rescaled
+      // after the PV product of tile i-1, whose probabilities still have the
+      // old reference.  Masks and moves are out of line (settle): few tiles
+      // have either.
+      auto settle = [&] {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const bool valid = (vmask >> ((e >> 2) * 16 + kbase + 2 * (e & 3))) & 1u;
+          d[e] = valid ? d[e] : -INFINITY;
+          mx = fmaxf(mx, valid ? st.s[e >> 2][e & 3] * c : -INFINITY);
+        }
+        bool over = false;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) over |= d[e] > kRescaleSlack;
+        if (__ballot(over) != 0) {  // wave-uniform
+          mx = max_lane_groups(mx);
+          const float m_new = fmaxf(m_run, mx);
+          alpha = m_run == -INFINITY ? 0.f : fast_exp2(m_run - m_new);
+          m_run = m_new;
+          moved = true;
+          l_run *= alpha;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const bool valid = (vmask >> ((e >> 2) * 16 + kbase + 2 * (e & 3))) & 1u;
+            d[e] = valid ? __builtin_fmaf(st.s[e >> 2][e & 3], c, -m_run) : -INFINITY;
+          }
+        }
+      };
+      auto softmax_step = [&](auto U) {
+        constexpr int w = decltype(U)::value - kSettle;
+        if constexpr (w >= 0 && w < kSoftmaxSteps) {
+          if constexpr (w < 2) {
+            if constexpr (w == 0) scores_settled<1>(st.s);
+#pragma unroll
+            for (int e = 4 * w; e < 4 * w + 4; ++e) d[e] = __builtin_fmaf(st.s[w][e & 3], c, -m_run);
+          } else if constexpr (w == 2) {
+            x[0] = fmaxf(fmaxf(d[0], d[1]), d[2]);
+            x[0] = fmaxf(fmaxf(x[0], d[3]), d[4]);
+          } else if constexpr (w == 3) {
+            x[0] = fmaxf(fmaxf(x[0], d[5]), d[6]);
+            x[0] = fmaxf(x[0], d[7]);
+          } else if constexpr (w == 4) {
+            moved = false;
+            if (vmask != 0xffffffffu || __ballot(x[0] > kRescaleSlack) != 0) settle();
+          } else {
+            constexpr int e = (w - 5) / 7 * 2, j = (w - 5) % 7;  // elements e, e + 1
+            if constexpr (j < 2) {
+              x[j] = fast_exp2(d[e + j]);
+            } else if constexpr (j == 2) {
+              psum = (e == 0 ? 0.f : psum) + x[0];
+              psum += x[1];
+            } else if constexpr (j == 3) {
+              const bf16x2 hi = {(__bf16)x[0], (__bf16)x[1]};
+              n_hi[e / 2] = __builtin_bit_cast(uint32_t, hi);
+            } else if constexpr (j == 4) {
+              x[0] -= __uint_as_float(n_hi[e / 2] << 16);
+            } else if constexpr (j == 5) {
+              x[1] -= __uint_as_float(n_hi[e / 2] & 0xffff0000u);
+            } else {
+              const bf16x2 lo = {(__bf16)x[0], (__bf16)x[1]};
+              n_lo[e / 2] = __builtin_bit_cast(uint32_t, lo);
+              if constexpr (e == 6) l_run += psum;
+            }
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // a step stays where it stands
+      };
+      auto qk_side = [&](int i, auto I) {
+        constexpr int n = decltype(I)::value;
+        if constexpr (n <= R::kRows) piece(i + 2, I);
+        // the id of tile i+3: in flight between two items' reads, complete
+        // once the later item's wait is
+        if constexpr (n == 10)
+          asm volatile("ds_read_b32 %0, %1"
+                       : "=&v"(id)
+                       : "v"(id0 + min(i + 3, L::kRingTiles - 1) * kKeysPerTile * 4)
+                       : "memory");
+        if constexpr (n == 11 + kAhead) {
+          asm volatile("" : "+v"(id));
+          id = i + 3 < n_tiles ? id : -1;
+        }
+        if constexpr (n == kQkItems - 1) vmask = __builtin_amdgcn_readlane(tile_masks, i);
+      };
+      wait_vmcnt<R::kLoads>();
       __builtin_amdgcn_s_barrier();
-      if (2 < n_tiles) {
-        fire_tile(2, tile_src(2));
-        fired = 2;
+      tile_items<0, kQkItems>(addr(0), qreg, acc, st, [&](auto I) { qk_side(0, I); }, [](auto) {});
+      scores_settled<16>(st.s);
+      for_each_int<kSettle + kSoftmaxSteps>(softmax_step);
+      st.p_hi = n_hi;
+      st.p_lo = n_lo;
+      for (int i = 1; i < n_tiles; ++i) {
+#pragma unroll
+        for (int k = 0; k < 32; ++k) asm volatile("" : "+a"(acc[k]));  // see rescale
+        src = key_src(id);
+        wait_vmcnt<R::kLoads>();
+        __builtin_amdgcn_s_barrier();
+        tile_items<0, kItems>(addr(i), qreg, acc, st, [&](auto I) { qk_side(i, I); }, softmax_step);
+        if (moved) rescale(acc, alpha);
+        st.p_hi = n_hi;
+        st.p_lo = n_lo;
       }
+      tile_items<kQkItems, kItems>(addr(n_tiles), qreg, acc, st, [](auto) {}, [](auto) {});
+      accumulators_settled(acc);
     }
-    for (int j = 0; j < n_tiles; ++j) {
-      wait_own(j);
-      __builtin_amdgcn_s_barrier();  // X_j
-      fused(j, sb);
-      if (team_b && j + 1 < n_tiles) wait_own(j + 1);
-      __builtin_amdgcn_s_waitcnt(0xC07F);
-      __builtin_amdgcn_s_barrier();  // Y_j
-      if (team_b && j + 3 < n_tiles) {
-        fire_tile(j + 3, tile_src(j + 3));
-        fired = j + 3;
-      }
-      softmax(sb, __builtin_amdgcn_readlane(tile_masks, j), p_hi, p_lo);
-      // team A issues its share of tile j+2 here, where it waits for team B's
-      // QK/PV anyway, not between X_j and its own QK/PV
-      if (!team_b && j + 2 < n_tiles) {
-        fire_tile(j + 2, tile_src(j + 2));
-        fired = j + 2;
-      }
-    }
-    if (!team_b) __builtin_amdgcn_s_barrier();
+    wait_vmcnt<0>();  // the zero rows past the last tile: no DMA outlives the workgroup
   } else {
-    int next_refill = 16;  // the next tile index whose issue triggers a slot-id refill
-    for (int i = 0; i < n_tiles; ++i) {
-      wait_tile(i);
-      __builtin_amdgcn_s_barrier();  // every wave's share of tile i landed
-      // stage offsets: tile i, and tile i-1 (whose stage receives tile i+3)
-      const int st_cur = (i & (kStages - 1)) * kStageBytes;
-      const int st_prev = ((i + kStages - 1) & (kStages - 1)) * kStageBytes;
-      const char *st_ckv = lds + st_cur;
-      f32x4 sacc[2];
-      if constexpr (FS == 1) {
-        // S^T of tile i fused with the PV product of tile i-1 (tile 0: the PV
-        // part reads the zeroed stage with zero probabilities)
+    bf16x8 p_hi = {}, p_lo = {};
+    auto lds_addr = [](const char *q) {
+      return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)q;
+    };
+    const int k0 = key_of_row(r16), k1 = 16 + key_of_row(r16);
+    if constexpr (kTeams) {
+      const bool team_b = wave >= 4;
+      f32x4 sb[2];  // S^T of the wave's current tile, from its QK/PV step to its softmax
+      auto fused = [&](int i, f32x4 (&sacc)[2]) {
+        const char *st_ckv = lds + (i & (kStages - 1)) * kStageBytes;
+        const char *st_prev = lds + ((i + kStages - 1) & (kStages - 1)) * kStageBytes;
         const char *st_kpe = st_ckv + kCkvStageBytes;
         const FusedAddr fa = {
             lds_addr(st_ckv + ring_row(k0) * kCkvPitch + g * 16), lds_addr(st_ckv + ring_row(k1) * kCkvPitch + g * 16),
             lds_addr(st_kpe + kpe_group_off(k0 >> 3) + (k0 & 7) * 16 + g * 128),
             lds_addr(st_kpe + kpe_group_off(k1 >> 3) + (k1 & 7) * 16 + g * 128),
-            lds_addr(lds + st_prev + ring_row(kbase + 2 * (r16 >> 2)) * kCkvPitch + 4 * (r16 & 3) * 2)};
+            lds_addr(st_prev + ring_row(kbase + 2 * (r16 >> 2)) * kCkvPitch + 4 * (r16 & 3) * 2)};
         qk_pv_tile(fa, qreg, p_hi, p_lo, acc, sacc);
-      } else {
-        scores(st_ckv, sacc);
-        if (i > 0) pv(lds + st_prev, p_hi, p_lo);
-      }
-      if (FS >= 2) xput(sacc[0]);
-      // (The one-slice layouts compute the addresses after the barrier: their
-      // waves have no registers to hold them across it.)
-      const bool refill_stage = i + kStages - 1 < n_tiles;
-      TileSrc nxt;
-      if (FS >= 2 && refill_stage) nxt = tile_src(i + kStages - 1);
-      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): partial written, tile i-1 read
-      __builtin_amdgcn_s_barrier();
-      if (FS == 1 && refill_stage) nxt = tile_src(i + kStages - 1);
-      if (refill_stage) fire_tile(i + kStages - 1, nxt);
-      // Ring refill (layouts whose ring holds 32 tiles' ids): once tile J = 16 m
-      // (m >= 1) is issued, every wave has passed a barrier since it read the
-      // ids of tiles J - 16 .. J - 1, so their half of the ring takes the ids of
-      // tiles J + 16 .. J + 31 (one 4-byte DMA per lane; raw ids, checked when
-      // issued).  The DMA completes before the loads of tile J + 1 (in-order
-      // vmcnt) and is visible after that tile's barrier, 14 iterations before
-      // tile J + 16 is issued.  The stage waits meanwhile count one extra load,
-      // which only makes them wait longer.
-      if constexpr (FS >= 2) {
-        static_assert(W == 8, "a half refill is 512 ids, one per lane of 8 waves");
-        const int J = i + kStages - 1;
-        if (J == next_refill) {  // J = 16, 32, ... (kept in a scalar, not tested per tile)
-          next_refill += 16;
-          if (J + 16 < n_tiles) {
-            const int key = (J + 16) * kKeysPerTile + wave * 64 + lane;  // W == 8: 512 keys
-            const int32_t *src = key < n_keys ? p.idx + (int64_t)t * p.idx_st + k_begin + key
-                                              : g_minus_one + lane;
-            lds_dma4(src, slots + ((J + 16) % L::kRingTiles) * kKeysPerTile + wave * 64);
-          }
+      };
+      // Both teams run the same loop (X_j, fused j, Y_j, softmax j); team B
+      // passes one extra barrier first and team A one after, so the barriers
+      // pair A's X_j with B's Y_{j-1} and A's Y_j with B's X_j: each team's
+      // QK/PV of a tile runs while the other team does its softmax.  Before a
+      // barrier that lets either team compute tile j, both teams' shares of
+      // tile j have landed: A waits before X_j, B before Y_{j-1}.  The stage of
+      // tile j-2 is free once both teams passed their fused step j-1, i.e.
+      // after the pair (A's X_j, B's Y_{j-1}): B fires its share of tile j+2
+      // right after that pair (before its softmax of tile j-1), A after its
+      // softmax of tile j (while B runs its fused step j).
+      int fired = pre - 1;  // last tile whose share this wave has issued
+      auto wait_own = [&](int j) {  // this wave's share of tile j landed
+        const int ahead = fired - j;
+        if (ahead >= 2)
+          wait_vmcnt<2 * R::kLoads>();
+        else if (ahead == 1)
+          wait_vmcnt<R::kLoads>();
+        else
+          wait_vmcnt<0>();
+      };
+      if (team_b) {
+        // this barrier is team A's X_0: team B's share of tile 0 lands first
+        wait_own(0);
+        __builtin_amdgcn_s_barrier();
+        if (2 < n_tiles) {
+          fire_tile(2, tile_src(2));
+          fired = 2;
         }
       }
-      if (FS >= 2) reduce(sacc);
-      softmax(sacc, __builtin_amdgcn_readlane(tile_masks, i), p_hi, p_lo);
+      for (int j = 0; j < n_tiles; ++j) {
+        wait_own(j);
+        __builtin_amdgcn_s_barrier();  // X_j
+        fused(j, sb);
+        if (team_b && j + 1 < n_tiles) wait_own(j + 1);
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        __builtin_amdgcn_s_barrier();  // Y_j
+        if (team_b && j + 3 < n_tiles) {
+          fire_tile(j + 3, tile_src(j + 3));
+          fired = j + 3;
+        }
+        softmax(sb, __builtin_amdgcn_readlane(tile_masks, j), p_hi, p_lo);
+        // team A issues its share of tile j+2 here, where it waits for team B's
+        // QK/PV anyway, not between X_j and its own QK/PV
+        if (!team_b && j + 2 < n_tiles) {
+          fire_tile(j + 2, tile_src(j + 2));
+          fired = j + 2;
+        }
+      }
+      if (!team_b) __builtin_amdgcn_s_barrier();
+    } else {
+      int next_refill = 16;  // the next tile index whose issue triggers a slot-id refill
+      for (int i = 0; i < n_tiles; ++i) {
+        wait_tile(i);
+        __builtin_amdgcn_s_barrier();  // every wave's share of tile i landed
+        // stage offsets: tile i, and tile i-1 (whose stage receives tile i+3)
+        const int st_cur = (i & (kStages - 1)) * kStageBytes;
+        const int st_prev = ((i + kStages - 1) & (kStages - 1)) * kStageBytes;
+        const char *st_ckv = lds + st_cur;
+        f32x4 sacc[2];
+        scores(st_ckv, sacc);
+        if (i > 0) pv(lds + st_prev, p_hi, p_lo);
+        xput(sacc[0]);
+        const bool refill_stage = i + kStages - 1 < n_tiles;
+        TileSrc nxt;
+        if (refill_stage) nxt = tile_src(i + kStages - 1);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): partial written, tile i-1 read
+        __builtin_amdgcn_s_barrier();
+        if (refill_stage) fire_tile(i + kStages - 1, nxt);
+        // Ring refill (layouts whose ring holds 32 tiles' ids): once tile J = 16 m
+        // (m >= 1) is issued, every wave has passed a barrier since it read the
+        // ids of tiles J - 16 .. J - 1, so their half of the ring takes the ids of
+        // tiles J + 16 .. J + 31 (one 4-byte DMA per lane; raw ids, checked when
+        // issued).  The DMA completes before the loads of tile J + 1 (in-order
+        // vmcnt) and is visible after that tile's barrier, 14 iterations before
+        // tile J + 16 is issued.  The stage waits meanwhile count one extra load,
+        // which only makes them wait longer.
+        {
+          static_assert(FS >= 2 && W == 8, "a half refill is 512 ids, one per lane of 8 waves");
+          const int J = i + kStages - 1;
+          if (J == next_refill) {  // J = 16, 32, ... (kept in a scalar, not tested per tile)
+            next_refill += 16;
+            if (J + 16 < n_tiles) {
+              const int key = (J + 16) * kKeysPerTile + wave * 64 + lane;  // W == 8: 512 keys
+              const int32_t *src = key < n_keys ? p.idx + (int64_t)t * p.idx_st + k_begin + key
+                                                : g_minus_one + lane;
+              lds_dma4(src, slots + ((J + 16) % L::kRingTiles) * kKeysPerTile + wave * 64);
+            }
+          }
+        }
+        reduce(sacc);
+        softmax(sacc, __builtin_amdgcn_readlane(tile_masks, i), p_hi, p_lo);
+      }
     }
+    if (n_tiles > 0) pv(lds + ((n_tiles - 1) & (kStages - 1)) * kStageBytes, p_hi, p_lo);
   }
-  if (n_tiles > 0) pv(lds + ((n_tiles - 1) & (kStages - 1)) * kStageBytes, p_hi, p_lo);
 
   // ---- epilogue: lanes of a head hold partial sums over disjoint keys
   l_run += __shfl_xor(l_run, 16);
@@ -1178,26 +1527,6 @@ static_assert(kWaveLds <= 160 * 1024, "LDS budget of one gfx950 CU");
 // the merge after the loop reuses each wave's ring: three 8 KB slices (one
 // per other wave), then 16 (m, l) pairs
 static_assert(3 * 8192 + 16 * 8 <= kWaveRing, "merge space");
-
-// The rare rescaling of the four-wave kernel's O^T accumulators, which live in AGPRs.  The empty
-// asm statements pin them there around it: left to itself the compiler copies
-// all of them to VGPRs at the head of every loop iteration, ready for this
-// branch -- 128 moves per 16-key block, and the registers they take push Q^T
-// into AGPRs, which costs four more moves before most QK MFMAs (2048 prefill
-// tokens 417 -> 350 us, 300 tokens 104 -> 84).
-template <int N>
-__device__ __forceinline__ void rescale(f32x4 (&acc)[N], float alpha) {
-#pragma unroll
-  for (int i = 0; i < N; ++i) asm volatile("" : "+a"(acc[i]));
-#pragma unroll
-  for (int i = 0; i < N; ++i) acc[i] *= alpha;
-#pragma unroll
-  for (int i = 0; i < N; ++i) asm volatile("" : "+a"(acc[i]));
-}
-
-__device__ __forceinline__ uint32_t lds_u32(const char *p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p;
-}
 
 template <bool NARROW>
 __global__ __launch_bounds__(kWaveWaves * 64, 1) void dsa_attn_wave_kernel(AttnParams p) {
@@ -1763,12 +2092,17 @@ hipError_t launch_attention_partial(const AttnParams &p, hipStream_t stream) {
   if (attn_wave_layout(p.T, p.H, p.num_splits)) return launch_wave(p, groups, stream);
   if (groups % 8 == 0) {
     // Four-wave workgroups of four head groups each -- twice the workgroups
-    // of the eight-wave layout, each gathering the chunk's keys -- finish
-    // sooner while that grid fits the CUs in one round (H=128, top-k 2048:
-    // T=16 with 8 splits 35.1 us against 41.7 us for eight-wave workgroups
-    // and 16 splits, T=32 with 4 splits 49.6 against 53.0 us; the same
-    // bits); past that the eight-wave workgroups' shared gathers win.
-    if ((int64_t)p.T * p.num_splits * (groups / 4) <= kNumCU)
+    // of the eight-wave layout, each gathering the chunk's keys for about 0.6
+    // of its time -- finish sooner while that grid fits the CUs in one round
+    // (H=128, top-k 2048: T=16 32 us against 42 us for eight-wave workgroups
+    // and 16 splits, T=32 43 against 53 us), and in three rounds where the
+    // eight-wave grid takes two (T=86 130 against 144 us, T=100 136 against
+    // 147; T=125 at top-k 1024 109 both).  With one or two chunks the shared
+    // gathers count for more: T=190, top-k 512 97 against 94 us, 300 tokens of
+    // a prompt 52 against 45; in two rounds against one T=128 131 against 121.
+    // The same bits either way.
+    const int64_t blocks = (int64_t)p.T * p.num_splits * (groups / 4);
+    if (blocks <= kNumCU || (p.num_splits >= 3 && blocks > 2 * kNumCU && blocks <= 3 * kNumCU))
       return launch_ring<4, 1>(p, groups / 4, stream);
     return launch_ring<8, 1>(p, hb, stream);  // one wave per head group
   }

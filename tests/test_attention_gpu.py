@@ -690,3 +690,44 @@ def test_rows_padded_at_their_end(H, T, splits):
     _assert_parity(out, lse, *_oracle(d), f"padded rows H={H} splits={splits}")
     empty = [t for t in range(T) if bool((idx[t] < 0).all())]
     assert empty and torch.isneginf(lse[empty]).all() and (out[empty] == 0).all()
+
+
+# The four-wave ring layout (H = 64; H = 128 with a grid of one round, and of
+# three where the eight-wave one takes two: T=90 with 3 chunks): rows whose
+# scores rise (even heads) or fall (odd heads) by about 150 log2 units, so the
+# reference max moves every few tiles, tiles that are padding throughout, at
+# the front and inside, and lengths of one, two and three tiles and past them.
+# paged: pages further apart than their rows, gathered at 64-bit addresses.
+@pytest.mark.parametrize("H,T,K,splits,paged", [(64, 9, 2048, 1, False), (64, 9, 2048, 1, True),
+                                                (64, 9, 1000, 3, False), (128, 9, 2048, 4, True),
+                                                (128, 90, 512, 0, False)])
+def test_four_wave_ring_moving_reference(H, T, K, splits, paged):
+    slots, page = 4096, 64
+    d = workloads.attention_inputs(T, H, K, slots // page, page, 7 * H + T)
+    g = d.pop("gen")
+    ramp = torch.arange(slots, dtype=torch.float32) / slots
+    d["kpe_cache"].view(slots, -1)[:, 0] = (ramp * 60).to(torch.bfloat16)
+    d["q_pe"][:, :, 0] = 16.0
+    d["q_pe"][:, 1::2, 0] = -16.0
+    idx = torch.full((T, K), -1, dtype=torch.int32)
+    for t in range(T):
+        n = [K, 32, 33, 64, 65, 96, 97, 128, K - 1][t % 9]
+        idx[t, :n] = torch.randperm(slots, generator=g)[:n].sort().values.to(torch.int32)
+        if t % 2 == 1:
+            idx[t, :min(32, n - 1)] = -1
+        if t % 3 == 0:
+            idx[t, 64:96] = -1
+    d.update(sparse_indices=idx, sm_scale=workloads.SM_SCALE)
+    ref = _oracle(d)
+    dev = workloads.to_device({k: d[k] for k in ("q_nope", "q_pe", "ckv_cache", "kpe_cache", "sparse_indices")}, DEV)
+    if paged:
+        for name in ("ckv_cache", "kpe_cache"):
+            c = dev[name]
+            apart = torch.zeros((c.shape[0], 2) + tuple(c.shape[1:]), dtype=c.dtype, device=DEV)
+            apart[:, 0] = c
+            dev[name] = apart[:, 0]
+    print(f"moving reference H={H} T={T} K={K} splits={splits} paged={paged}", flush=True)
+    args = (dev["q_nope"], dev["q_pe"], dev["ckv_cache"], dev["kpe_cache"], dev["sparse_indices"], d["sm_scale"])
+    out, lse = kernel_splitk(*args, SPLIT_K=splits) if splits else kernel(*args)
+    torch.cuda.synchronize()
+    _assert_parity(out.cpu(), lse.cpu(), *ref, f"moving reference H={H} T={T} paged={paged}")
