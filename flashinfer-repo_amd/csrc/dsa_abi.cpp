@@ -76,7 +76,7 @@ void choose_splits(int64_t T, int64_t H, int64_t K, int32_t requested, int32_t *
     int64_t max_s;
     // the four-wave layout while it gets at least 2 splits (at least 4 for
     // multiples of 8 groups, whose four-wave ring layout is faster at 2:
-    // H=128 T=16 35.1 us with 8 splits against 36.8 us)
+    // H=128 T=16 32 us with 8 splits against 36.8 us)
     if (groups % 2 != 0 || Tn * groups <= dsa::kNumCU / (groups % 8 == 0 ? 4 : 2)) {
       // four-wave layout, T x S x groups workgroups within one round
       S = dsa::kNumCU / (Tn * groups);
