@@ -598,7 +598,7 @@ __device__ __forceinline__ void pv_mfma(f32x4 &acc, const bf16x8 &av, const u32x
 }
 // At least STATES wait states between item_qk's last MFMA and the first read
 // of its result (16 are more than an MFMA of this shape asks for; in the
-// stream kSettle + 1 PV MFMAs, four states each, stand in between as well).
+// stream kSettle PV MFMAs, four states each, stand in between as well).
 template <int STATES>
 __device__ __forceinline__ void scores_settled(f32x4 (&s)[2]) {
   asm volatile("s_nop %2" : "+v"(s[0]), "+v"(s[1]) : "n"(STATES - 1));
