@@ -1543,12 +1543,15 @@ __global__ __launch_bounds__(kWaveWaves * 64, 1) void dsa_attn_wave_kernel(AttnP
   const int k_begin = split * p.chunk;
   const int n_keys = max(0, min(p.K, k_begin + p.chunk) - k_begin);
   const int n_blocks = (n_keys + kWaveBlock - 1) / kWaveBlock;
-  // This wave's blocks.  Few blocks: wave, wave + 4, ..., so that padding at a
-  // row's end falls to all four waves alike.  Long runs, which are sorted: a
-  // quarter each, of the blocks up to the row's last valid id (with every
-  // fourth block a wave meets each cache page in more pieces: 2048 prefill
-  // tokens 424 us against 417).
-  const bool sorted = n_blocks >= kWaveWaves * kWaveSortBlocks;
+  // This wave's blocks: a quarter of the chunk's, one after the other, so a
+  // wave adds up one run of keys in the row's order.  (Every fourth block
+  // instead is another order of the fp32 sums; it gains 1 % for 64 decode
+  // tokens, 29.5 against 29.9 us, and loses 2 % where the runs are sorted: 2048
+  // prefill tokens 424 us against 417.)  Few blocks keep the given order and
+  // only leave out the padding after the quarter's last valid id; long runs are
+  // sorted, and divided anew where padding ends the row.
+  const int quarter = n_blocks * (wave + 1) / kWaveWaves - n_blocks * wave / kWaveWaves;
+  const bool sorted = quarter >= kWaveSortBlocks;
   int my_blocks = 0;
   char *ring = lds + wave * kWaveRing;
 
@@ -1557,8 +1560,6 @@ __global__ __launch_bounds__(kWaveWaves * 64, 1) void dsa_attn_wave_kernel(AttnP
   // issued, and Q^T is read into registers from the staging.
   constexpr int kPer = kWaveIds / (kWaveWaves * 64);  // ids per lane (a wave takes <= 512 keys)
   const int32_t *isrc = p.idx + (int64_t)t * p.idx_st + k_begin;
-  const int all_blocks = (n_blocks - wave + kWaveWaves - 1) / kWaveWaves;  // unsorted
-  const int n_mine = all_blocks * kWaveBlock;
   int sv[kPer];
   // the ids of the quarter of the first `keys` keys
   auto load_quarter = [&](int keys) {
@@ -1572,45 +1573,13 @@ __global__ __launch_bounds__(kWaveWaves * 64, 1) void dsa_attn_wave_kernel(AttnP
     }
     return k0;
   };
-  int k0 = 0;
-  if (sorted) {
-    k0 = load_quarter(n_keys);
-  } else {
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-      const int i = k * 64 + lane;
-      const int key = ((i >> 4) * kWaveWaves + wave) * kWaveBlock + (i & 15);
-      sv[k] = i < n_mine && key < n_keys ? isrc[key] : -1;
-    }
-  }
+  const int k0 = load_quarter(n_keys);
   auto valid_id = [&](int s) { return (s >= 0 && (int64_t)s < p.num_slots) ? s : -1; };
 
   int32_t *my_ids = slots + wave * (kWaveIds / kWaveWaves);
-  if (!sorted) {
-    // few blocks: the keys keep their given order (the sort below costs
-    // about 1 us of the prologue and pays only on long runs)
-#pragma unroll
-    for (int k = 0; k < kPer; ++k)
-      if (k * 64 < n_mine) {  // wave-uniform
-        const int id = valid_id(sv[k]);
-        my_ids[k * 64 + lane] = id;
-        const uint64_t m = __ballot(id >= 0);
-        if (m != 0) my_blocks = (k * 64 + 63 - __builtin_clzll(m)) / kWaveBlock + 1;
-      }
-  } else {
-    // ---- order this wave's keys by slot: a stable counting sort on the top 8
-    // bits of the slot id (256 buckets, each a contiguous range of the cache),
-    // in the wave's own (not yet used) ring, so no workgroup barrier is
-    // needed: one wave's LDS accesses execute in program order.  Every wave of
-    // every workgroup then sweeps the cache upwards at the same time, which
-    // keeps address translation and cache lines shared between neighbouring
-    // gathers.  The order depends on the ids alone: results stay
-    // deterministic.  Padding takes no place; where some of it ends the row the
-    // waves divide the keys before it anew (the places of their last valid ids
-    // meet in the ring of wave 0).  Scratch: per-vector bucket counts hist[k][256] (bytes;
-    // vector k = keys 64k .. 64k+63 of the wave), their start positions
-    // start[k][256] (u16); the sorted ids go to the wave's 512-entry slice of
-    // the id array.
+  if (n_blocks > kWaveWaves * (kWaveSortBlocks - 1)) {  // some wave sorts
+    // Where padding ends the row, the waves divide the keys before it anew (the
+    // places of their last valid ids meet in the ring of wave 0).
     int last = -1;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
@@ -1623,6 +1592,30 @@ __global__ __launch_bounds__(kWaveWaves * 64, 1) void dsa_attn_wave_kernel(AttnP
     last = max(max(lasts[0], lasts[1]), max(lasts[2], lasts[3]));
     last = __builtin_amdgcn_readfirstlane(last);
     if (last + 1 < n_keys) load_quarter(last + 1);
+  }
+  if (!sorted) {
+    // few blocks: the keys keep their given order (the sort below costs
+    // about 1 us of the prologue and pays only on long runs)
+    constexpr int kIds = kWaveSortBlocks * kWaveBlock / 64;  // vectors of a quarter of at most that many blocks
+#pragma unroll
+    for (int k = 0; k < kIds; ++k) {
+      const int id = valid_id(sv[k]);  // (-1 past the quarter)
+      my_ids[k * 64 + lane] = id;
+      const uint64_t m = __ballot(id >= 0);
+      if (m != 0) my_blocks = (k * 64 + 63 - __builtin_clzll(m)) / kWaveBlock + 1;
+    }
+  } else {
+    // ---- order this wave's keys by slot: a stable counting sort on the top 8
+    // bits of the slot id (256 buckets, each a contiguous range of the cache),
+    // in the wave's own (not yet used) ring, so no workgroup barrier is
+    // needed: one wave's LDS accesses execute in program order.  Every wave of
+    // every workgroup then sweeps the cache upwards at the same time, which
+    // keeps address translation and cache lines shared between neighbouring
+    // gathers.  The order depends on the ids alone: results stay
+    // deterministic.  Padding takes no place.  Scratch: per-vector bucket counts
+    // hist[k][256] (bytes; vector k = keys 64k .. 64k+63 of the wave), their start
+    // positions start[k][256] (u16); the sorted ids go to the wave's 512-entry
+    // slice of the id array.
     uint8_t *hist = (uint8_t *)ring;
     uint16_t *start = (uint16_t *)(ring + kPer * 256);
     static_assert(kPer * 256 * 3 <= kWaveRing, "sort scratch in the ring");

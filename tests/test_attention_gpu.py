@@ -731,3 +731,23 @@ def test_four_wave_ring_moving_reference(H, T, K, splits, paged):
     out, lse = kernel_splitk(*args, SPLIT_K=splits) if splits else kernel(*args)
     torch.cuda.synchronize()
     _assert_parity(out.cpu(), lse.cpu(), *ref, f"moving reference H={H} T={T} paged={paged}")
+
+
+# One chunk of few blocks (the automatic splits of small batches): the lowest and
+# a middle count of blocks, the last one that no wave sorts, and several chunks.
+@pytest.mark.parametrize("chunk,splits", [(128, 1), (384, 1), (896, 1), (256, 8)])
+def test_a_wave_adds_up_one_run_of_keys_in_row_order(chunk, splits):
+    """With equal probabilities, the first quarter's values of +2^20 and -2^20
+    cancel exactly inside one wave, and the third quarter's 2^-12 stay whole
+    in another: a sum that meets both in one fp32 accumulator loses them."""
+    K, page, v = chunk * splits, 64, 2.0 ** -12
+    val = torch.zeros(chunk)
+    val[:chunk // 8], val[chunk // 8:chunk // 4] = 2.0 ** 20, -(2.0 ** 20)
+    val[chunk // 2:3 * chunk // 4] = v
+    ckv = val.repeat(splits).to(torch.bfloat16)[:, None].expand(K, 512).reshape(K // page, page, 512).contiguous()
+    d = _dict(torch.zeros(2, 16, 512, dtype=torch.bfloat16), torch.zeros(2, 16, 64, dtype=torch.bfloat16), ckv,
+              torch.zeros(K // page, page, 64, dtype=torch.bfloat16),
+              torch.arange(K, dtype=torch.int32).repeat(2, 1), 1.0)
+    print(f"one run per wave: chunk={chunk} splits={splits}", flush=True)
+    out, _ = _run(kernel_splitk, d, SPLIT_K=splits)
+    assert (out.float() == v / 4).all(), out.float().unique()
