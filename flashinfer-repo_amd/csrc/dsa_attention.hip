@@ -1522,7 +1522,11 @@ constexpr int kWaveStage = kWaveKpeOff + kWaveBlock * 128;  // + 2048 = 18944
 constexpr int kWaveRing = 2 * kWaveStage;
 constexpr int kWaveIds = kMaxChunkWide;                 // slot ids of a chunk, staged once
 constexpr int kWaveSortBlocks = 16;  // a wave sorts its keys by slot from this many blocks on
-constexpr int kWaveLds = kWaveWaves * kWaveRing + kWaveIds * 4;
+// After the rings: the slot ids, then the place of each wave's last valid id.
+// Those four words are read behind one barrier while other waves run on, so
+// they share their place with nothing.
+constexpr int kWaveLastOff = kWaveWaves * kWaveRing + kWaveIds * 4;
+constexpr int kWaveLds = kWaveLastOff + kWaveWaves * 4;
 static_assert(kWaveLds <= 160 * 1024, "LDS budget of one gfx950 CU");
 // the merge after the loop reuses each wave's ring: three 8 KB slices (one
 // per other wave), then 16 (m, l) pairs
@@ -1578,15 +1582,14 @@ __global__ __launch_bounds__(kWaveWaves * 64, 1) void dsa_attn_wave_kernel(AttnP
 
   int32_t *my_ids = slots + wave * (kWaveIds / kWaveWaves);
   if (n_blocks > kWaveWaves * (kWaveSortBlocks - 1)) {  // some wave sorts
-    // Where padding ends the row, the waves divide the keys before it anew (the
-    // places of their last valid ids meet in the ring of wave 0).
+    // Where padding ends the row, the waves divide the keys before it anew.
     int last = -1;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
       const uint64_t m = __ballot(valid_id(sv[k]) >= 0);
       if (m != 0) last = k0 + k * 64 + 63 - __builtin_clzll(m);
     }
-    int32_t *lasts = (int32_t *)(lds + kWaveRing - 16);
+    int32_t *lasts = (int32_t *)(lds + kWaveLastOff);
     if (lane == 0) lasts[wave] = last;
     lds_barrier();
     last = max(max(lasts[0], lasts[1]), max(lasts[2], lasts[3]));

@@ -751,3 +751,29 @@ def test_a_wave_adds_up_one_run_of_keys_in_row_order(chunk, splits):
     print(f"one run per wave: chunk={chunk} splits={splits}", flush=True)
     out, _ = _run(kernel_splitk, d, SPLIT_K=splits)
     assert (out.float() == v / 4).all(), out.float().unique()
+
+
+# One sorted chunk whose waves re-divide the keys before the padding: 61 blocks (the
+# fewest), all 128, and the last id in each wave's quarter.
+@pytest.mark.parametrize("H,K", [(16, 2048), (48, 2048), (16, 976)])
+def test_sorted_waves_divide_padded_rows_whatever_the_queries_hold(H, K):
+    """The waves exchange the place of the row's last valid id through LDS beside
+    the staging of Q.  Every q_pe word is the bits of a place far past the
+    row (0x3f803f80), so a place read from the staging would show."""
+    counts = [1, 16, 17, K // 4 - 1, K // 4 + 1, K // 2 + 3, 3 * K // 4 + 5, K - 1, K]
+    T, slots = 2 * len(counts), 4096
+    g = torch.Generator().manual_seed(H + K)
+    d = workloads.attention_inputs(T, H, K, slots // 64, 64, H + K)
+    d.pop("gen")
+    d["q_pe"].fill_(1.0)
+    idx = torch.full((T, K), -1, dtype=torch.int32)
+    for t in range(T):
+        n = counts[t % len(counts)]
+        idx[t, :n] = torch.randperm(slots, generator=g)[:n].to(torch.int32)
+    d.update(sparse_indices=idx, sm_scale=workloads.SM_SCALE)
+    print(f"re-divided rows H={H} K={K}", flush=True)
+    out, lse = _run(kernel_splitk, d, SPLIT_K=1)
+    _assert_parity(out, lse, *_oracle(d), f"re-divided rows H={H} K={K}")
+    for _ in range(3):
+        again = _run(kernel_splitk, d, SPLIT_K=1)
+        assert torch.equal(again[0], out) and torch.equal(again[1], lse)
