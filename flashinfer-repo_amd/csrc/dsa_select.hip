@@ -1067,6 +1067,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_estimates_kernel(In
     write_marked<KEYS>(p, sh, t, n, out, [](int i) { return i; });
     return;
   }
+  __syncthreads();  // every wave has read n_cand: mark_exact clears it
   // every candidate's exact score (estimates of zeros are), then the selection
   // from those
   if (!(band == 0.f)) {
@@ -1240,6 +1241,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_merge_kernel(Indexe
     write_marked<KEYS>(p, sh, t, KEYS, out, position);
     return;
   }
+  __syncthreads();  // every wave has read n_cand: mark_exact clears it
   // every listed position's exact score, then the selection from those
   if (!(band == 0.f)) {
     uint32_t *keys = (uint32_t *)row;

@@ -653,6 +653,32 @@ def test_selection_without_scores_of_hard_rows(kind, S):
         assert np.array_equal(got, want), kind
 
 
+# every instantiation of the row kernel and of the list merge
+@pytest.mark.parametrize("S,topk", [(3000, 512), (12000, 512), (32768, 512), (40000, 512), (140000, 1500), (262144, 2048)])
+def test_padded_batch_rows_take_the_first_positions(S, topk):
+    """Rows whose scores are all zero (padded rows of a batch: no weights or no
+    queries) tie everywhere, so the first top-k positions win; rows between
+    them are ordinary.  The rows' counts of open positions are cleared for a
+    second selection only once every wave has read them."""
+    T = 24
+    d = workloads.indexer_inputs(T=T, Hi=32, S=S, seed=S)
+    d["causal_limit"] = torch.full((T,), S - 1, dtype=torch.int32)
+    d["weights"][::3] = 0.0
+    d["q_idx"] = d["q_idx"].clone()
+    d["q_idx"][1::3] = 0
+    print(f"padded rows S={S}", flush=True)
+    got, want = _select_both(d, topk)
+    first = np.arange(topk, dtype=np.int32)
+    for t in range(T):
+        assert t % 3 == 2 or np.array_equal(got[t], first), t
+    assert np.array_equal(got, want)
+    g = workloads.to_device(d, DEV)
+    for _ in range(5):
+        again = run_indexer_and_topk(g["q_idx"], g["k_idx"], g["k_scale"], g["weights"], g["causal_limit"], topk)
+        torch.cuda.synchronize()
+        assert np.array_equal(again.cpu().numpy(), got)
+
+
 def test_selection_without_scores_after_nan_filled_lds():
     for S in (20000, 45000):
         d = _full_range(workloads.indexer_inputs(T=5, Hi=64, S=S, seed=77), torch.Generator().manual_seed(78))
