@@ -481,11 +481,17 @@ __device__ __forceinline__ void pick_digit(const uint32_t *tot, uint32_t prefix,
 // it needs after the VALU write of its SGPR source).
 extern "C" __device__ int amdgcn_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 
-// Keys whose place the register top-k decides by ranking them exactly: at most
-// this many; more take two more radix passes (exact keys) or exact scores for
-// the whole row (estimates).
+// Keys whose place the register top-k decides by ranking them: at most this
+// many; more are selected from by radix passes over their exact keys.
 constexpr int kMaxSurvivors = 256;
 constexpr int kMaxOpen = 512;
+// From estimates: with more open positions than kMaxBinOpen two more passes pin
+// the k-th estimate itself, so that only those within twice the bound of it stay
+// open, not those of its whole 16-bit bin (2^-7 of its value: where q and K share
+// a component, hundreds to thousands).  64 rows of 32768 positions with a shared
+// component four times the noise: 1393 us when a crowded bin was scored whole,
+// 60 now; ordinary rows have about 100 open and stay at 53.
+constexpr int kMaxBinOpen = 128;
 
 // Shared state of one top-k workgroup (KEYS = positions it holds).  One
 // space serves the radix histograms, then the row's q pieces, then the
@@ -500,6 +506,10 @@ struct TopkShared {
       int8_t qp[4 * 3 * 2 * kChunk];  // [head block][piece][k-step] MFMA A operands
       int8_t kp[4 * 3 * 2 * kChunk];  // [group of 16 positions][piece][k-step] B operands
       float4 r[kTopkThreads];         // relu'd dots, 1 KB per wave
+    };
+    struct {
+      int8_t qp_[4 * 3 * 2 * kChunk];  // (qp)
+      uint16_t open[KEYS];             // open places, ascending
     };
     int32_t pos[KEYS];
   };
@@ -706,6 +716,84 @@ __device__ __forceinline__ void exact_scores(const IndexerParams &p, Shared &sh,
     }
     __syncthreads();
   }
+}
+
+// The pieces of the lane's 2 x 16 codes at src (dims +0 and +64) as its operands.
+__device__ __forceinline__ void lane_pieces(const uint32_t *lut, const uint8_t *src, i32x4 (&k)[3][2]) {
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const uint4 r = *(const uint4 *)(src + 64 * ks);
+    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      uint32_t o[3];
+      pack_pieces4(lut[w[d] & 0xffu], lut[(w[d] >> 8) & 0xffu], lut[(w[d] >> 16) & 0xffu], lut[w[d] >> 24], o);
+#pragma unroll
+      for (int pc = 0; pc < 3; ++pc) k[pc][ks][d] = (int)o[pc];
+    }
+  }
+}
+
+// The same scores where there are more than a few groups: every wave takes a
+// group at a time on its own, so no barrier stands between rounds and the SIMD's
+// four waves hide each other's loads.  pos_of(i) is position i of the n, put(i,
+// score) takes its score.  NPC = 2: no third pieces in q and the group (every
+// magnitude below 32).  Bound by VALU work (table reads to pieces, the fp64 rounding
+// of the dots): 32768 positions 440 us (in the rounds above 1340).
+template <int NPC, typename Shared>
+__device__ __forceinline__ float group_score(const IndexerParams &p, const Shared &sh, const i32x4 (&k)[3][2],
+                                             float cs) {
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x & 63, g = lane >> 4;
+  const int nhb = p.Hi >> 4;
+  float G = 0.f;
+#pragma unroll 1
+  for (int h = 0; h < nhb; ++h) {
+    i32x4 C[2 * NPC - 1];
+#pragma unroll
+    for (int d = 0; d < 2 * NPC - 1; ++d) C[d] = i32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int a = 0; a < NPC; ++a) {
+        const i32x4 q = *(const i32x4 *)(sh.qp + ((h * 3 + a) * 2 + ks) * kChunk + lane * 16);
+#pragma unroll
+        for (int b = 0; b < NPC; ++b) C[a + b] = mfma(q, k[b][ks], C[a + b]);
+      }
+    const float *wl = sh.w + g * (p.Hi >> 2) + 4 * h;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      int hi = C[2][i];
+      if constexpr (NPC == 3) hi += (C[3][i] << 7) + (C[4][i] << 14);
+      G = __builtin_fmaf(wl[i], relu_dot(C[0][i] + (C[1][i] << 7), hi), G);
+    }
+  }
+  return sum_lane_groups(G) * cs;
+}
+
+template <typename Shared, typename PosOf, typename Put>
+__device__ __forceinline__ void exact_scores_many(const IndexerParams &p, Shared &sh, int n, PosOf pos_of, Put put) {
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int q_third = 0;
+#pragma unroll 1
+  for (int i = 0; i < (p.Hi >> 4) * 2; ++i) {
+    const i32x4 q = *(const i32x4 *)(sh.qp + (((i >> 1) * 3 + 2) * 2 + (i & 1)) * kChunk + lane * 16);
+    q_third |= q[0] | q[1] | q[2] | q[3];
+  }
+#pragma unroll 1
+  for (int i0 = wave * 16; i0 < n; i0 += kTopkThreads / 4) {
+    const int pos = pos_of(min(i0 + c, n - 1));
+    const float cs = p.k_cs[pos];
+    i32x4 k[3][2];
+    lane_pieces(sh.lut, p.k_codes + (int64_t)(pos >> 4) * p.k_code_stride + (pos & 15) * kIdxDim + g * 16, k);
+    int third = q_third;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) third |= k[2][j >> 2][j & 3];
+    const float score = __ballot(third != 0) == 0 ? group_score<2>(p, sh, k, cs) : group_score<3>(p, sh, k, cs);
+    if (lane < 16 && i0 + c < n) put(i0 + c, score);
+  }
+  __syncthreads();
 }
 
 // ---- the register top-k, one row per workgroup -----------------------------
@@ -1006,6 +1094,103 @@ __device__ __forceinline__ void store_row_pieces(const IndexerParams &p, Shared 
     store_pieces8(sh.lut, sh.qp + r.hb * (6 * kChunk), r.row, (threadIdx.x & 15) * 8, r.codes);
 }
 
+// Marks the keys that are taken for sure and lists the open ones: those within
+// band of the k-th key's bin [prefix, top], or, where they are many (see
+// kMaxBinOpen) and the band is a safe bound, within band of the k-th key
+// itself, which two more passes give (prefix == top then).  Returns how many
+// are open; `need` of the keys up to top, and the n_above open ones above it,
+// are among the k largest.  With the row's q pieces in the histograms' place.
+template <int EPT, typename Shared>
+__device__ __forceinline__ int mark_open(const IndexerParams &p, Shared &sh, const RowCodes &rc, int n,
+                                         const uint32_t (&key)[EPT], int phantom, float band, uint32_t &prefix,
+                                         uint32_t &top, uint32_t mask, int &need) {
+  top = prefix | 0xffffu;
+#pragma unroll 1
+  for (;;) {
+    mark_taken(sh, n, key, max(order_key(key_value(prefix) - band), 1u), order_key(key_value(top) + band), top);
+    store_row_pieces(p, sh, rc);
+    __syncthreads();
+    const int n_open = sh.n_cand;
+    if (!(band > 0.f) || n_open <= kMaxBinOpen || top == prefix) return n_open;  // uniform
+    __syncthreads();  // every wave has read n_cand
+    if (threadIdx.x == 0) sh.n_cand = sh.n_above = 0;
+#pragma unroll 1
+    for (int shift = 8; shift >= 0; shift -= 8)
+      radix_pass_regs(sh, sh.hist[0], false, shift, key, prefix, mask, need, phantom);
+    top = prefix;
+  }
+}
+
+// Exact scores of the listed open positions (at most kMaxOpen) in place of their
+// estimates: place_of(place) is a position.
+template <typename Shared, typename PosOf>
+__device__ __forceinline__ void score_listed(const IndexerParams &p, Shared &sh, int n_open, PosOf pos_of) {
+  if (n_open <= 64) {
+    exact_scores(p, sh, (n_open + 15) >> 4,
+                 [&](int b, int c) { return pos_of((int)sh.cand[min(b * 16 + c, n_open - 1)].y); },
+                 [&](int b, int c, float v) {
+                   if (b * 16 + c < n_open) sh.cand[b * 16 + c].x = max(order_key(v), 1u);
+                 });
+  } else {
+    exact_scores_many(p, sh, n_open, [&](int i) { return pos_of((int)sh.cand[i].y); },
+                      [&](int i, float v) { sh.cand[i].x = max(order_key(v), 1u); });
+  }
+}
+
+// More open keys than are listed (positions apart by less than the bound, or no
+// safe bound: all): the places of the keys in [lo, hi] among the first n go to
+// sh.open, as marks to sh.eqbits, and the keys above hi as marks to sh.bits.
+// Returns how many are open; `taken` how many are above.
+template <int EPT, typename Shared>
+__device__ __forceinline__ int list_open(Shared &sh, int n, const uint32_t (&key)[EPT], uint32_t lo, uint32_t hi,
+                                         int &taken) {
+  constexpr int kWords = EPT * kTopkThreads / 32, kWaves = kTopkThreads / 64;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) {
+    const uint64_t gb = __ballot(key[e] > hi);
+    const uint64_t ob = __ballot(key[e] >= lo) & ~gb;
+    if (lane == 0) {
+      sh.bits[e * kWaves + wave] = gb;
+      sh.eqbits[e * kWaves + wave] = ob;
+    }
+  }
+  __syncthreads();
+  const int nw = n - tid * 32;  // this word's places below n
+  uint32_t open = tid < kWords ? ((const uint32_t *)sh.eqbits)[tid] : 0u;
+  open &= nw >= 32 ? ~0u : (nw <= 0 ? 0u : (1u << nw) - 1u);
+  const int above = tid < kWords ? __builtin_popcount(((const uint32_t *)sh.bits)[tid]) : 0;
+  if (tid < kWords) ((uint32_t *)sh.eqbits)[tid] = open;
+  int total;
+  int o = block_exclusive_scan2(__builtin_popcount(open), above, sh.scan, &total, &taken).x;
+  while (open != 0) {
+    sh.open[o++] = (uint16_t)(tid * 32 + __builtin_ctz(open));
+    open &= open - 1;
+  }
+  __syncthreads();
+  return total;
+}
+
+// The keys for a selection from exact scores: open ones keep theirs, the taken
+// rank above all, the others below (as phantoms).
+template <int EPT, typename Shared>
+__device__ __forceinline__ void keep_open(const Shared &sh, uint32_t (&key)[EPT]) {
+  constexpr int kWaves = kTopkThreads / 64;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // (lane 2e + h holds half h of the wave's words of keys e)
+  const int word = ((min(lane, 2 * EPT - 1) >> 1) * kWaves + wave) * 2 + (lane & 1);
+  const int gw = ((const int *)sh.bits)[word], ow = ((const int *)sh.eqbits)[word];
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) {
+    const int g = (lane & 32) ? __builtin_amdgcn_readlane(gw, 2 * e + 1) : __builtin_amdgcn_readlane(gw, 2 * e);
+    const int o = (lane & 32) ? __builtin_amdgcn_readlane(ow, 2 * e + 1) : __builtin_amdgcn_readlane(ow, 2 * e);
+    key[e] = (g >> (lane & 31)) & 1 ? ~0u : (o >> (lane & 31)) & 1 ? key[e] : kPhantomKey;
+  }
+  __syncthreads();  // the marks are free
+}
+
 // Top-k of one row per workgroup from exact scores.
 template <int EPT>
 __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_kernel(IndexerParams p) {
@@ -1027,8 +1212,12 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_kernel(IndexerParam
 // lies within E of the estimates' bin, so keys more than 2 E above the bin are
 // taken, those more than 2 E below it are not, and the exact scores of the ones
 // between (a few dozen of 32768 ordinary scores) are computed here and ranked.
-// Where E is not a safe bound (huge, tiny or non-finite weights or scales) or
-// too many keys are open, the row's exact scores are computed and selected from.
+// A crowded bin is narrowed to the k-th estimate first (mark_open).  Where more
+// than kMaxOpen scores are still closer than E tells apart, or E is not a safe
+// bound (huge, tiny or non-finite weights or scales: all are open), the open
+// positions' exact scores replace their estimates in memory and the row is
+// selected from once more -- by this one workgroup: 64 rows of 32768
+// positions all tied at 0 take 490 us, of which a third are one same row 216.
 template <int EPT>
 __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_estimates_kernel(IndexerParams p) {
   constexpr int KEYS = EPT * kTopkThreads;
@@ -1051,34 +1240,31 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_estimates_kernel(In
   int need;
   find_bin(p, sh, key, KEYS - n, prefix, mask, need);
   const float band = sh.band;
-  mark_taken(sh, n, key, order_key(key_value(prefix) - band),
-             order_key(key_value(prefix | 0xffffu) + band), prefix | 0xffffu);
-  store_row_pieces(p, sh, rc);
-  __syncthreads();
-  const int n_open = sh.n_cand;
+  int phantom = KEYS - n;
+  uint32_t top;
+  int n_open = mark_open(p, sh, rc, n, key, phantom, band, prefix, top, mask, need);
   if (band == band && n_open <= kMaxOpen) {  // uniform
-    exact_scores(p, sh, (n_open + 15) >> 4,
-                 [&](int b, int c) { return (int)sh.cand[min(b * 16 + c, n_open - 1)].y; },
-                 [&](int b, int c, float v) {
-                   if (b * 16 + c < n_open) sh.cand[b * 16 + c].x = order_key(v);
-                 });
-    // (the keys above the bin that are open are not taken for sure)
+    score_listed(p, sh, n_open, [](int i) { return i; });
+    // (the keys above the bin, or the k-th, that are open are not taken for sure)
     rank_open(sh, n_open, need + sh.n_above);
     write_marked<KEYS>(p, sh, t, n, out, [](int i) { return i; });
     return;
   }
   __syncthreads();  // every wave has read n_cand: mark_exact clears it
-  // every candidate's exact score (estimates of zeros are), then the selection
-  // from those
-  if (!(band == 0.f)) {
-    exact_scores(p, sh, (n + 15) >> 4, [&](int b, int c) { return min(b * 16 + c, p.S - 1); },
-                 [&](int b, int c, float v) {
-                   if (b * 16 + c < n) row[b * 16 + c] = v;
-                 });
+  if (!(band == 0.f)) {  // (estimates of zeros are exact)
+    int taken;
+    const bool safe = band == band;  // else every position is open
+    const uint32_t lo = safe ? max(order_key(key_value(prefix) - band), 1u) : 0u;
+    const uint32_t hi = safe ? order_key(key_value(top) + band) : ~0u;
+    n_open = list_open(sh, n, key, lo, hi, taken);
+    exact_scores_many(p, sh, n_open, [&](int i) { return (int)sh.open[i]; },
+                      [&](int i, float v) { row[sh.open[i]] = v; });
     load_keys(row, p.S, key);
     to_keys(n, key);
+    keep_open(sh, key);
+    phantom = KEYS - n_open - taken;
   }
-  mark_exact(p, sh, n, key, KEYS - n);
+  mark_exact(p, sh, n, key, phantom);
   write_marked<KEYS>(p, sh, t, n, out, [](int i) { return i; });
 }
 
@@ -1090,8 +1276,9 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_estimates_kernel(In
 // row selects from the lists as the kernel above does from a row.  A list
 // takes the place of its chunk's estimates (all of a chunk's are in registers
 // by then): p.list_len order keys, 0 past the list's end, then their
-// positions, ascending.  A chunk whose bound is not safe, or whose list would
-// not fit, lists its k largest exact scores.  2 rows of 131071 positions, top-k
+// positions, ascending.  A chunk whose bound is not safe, or too many of whose
+// scores lie within the bound of the k-th, lists its k largest, by the exact
+// scores of those.  2 rows of 131071 positions, top-k
 // 2048: chunks 17 us, lists 20, against 235 for the four passes over exact
 // scores (one workgroup re-reading the row, its last pass uncoalesced).
 
@@ -1171,22 +1358,41 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_chunk_kernel(Indexe
   int need;
   find_bin(p, sh, key, KEYS - n, prefix, mask, need);
   const float band = sh.band;
-  const uint32_t lo = max(order_key(key_value(prefix) - band), 1u);
-  mark_taken(sh, n, key, ~0u, lo - 1, ~0u);  // every key from lo on
-  store_row_pieces(p, sh, rc);
-  __syncthreads();
-  int total = rank_marks<KEYS>(sh, n);
+  int phantom = KEYS - n, total;
+  uint32_t lo;
+  // every key from 2 E below the k-th key's bin on; where those do not fit, from
+  // 2 E below the k-th key itself, which two more passes give
+#pragma unroll 1
+  for (bool pinned = false;; pinned = true) {
+    lo = max(order_key(key_value(prefix) - band), 1u);
+    mark_taken(sh, n, key, ~0u, lo - 1, ~0u);
+    __syncthreads();
+    total = rank_marks<KEYS>(sh, n);
+    if (!(band > 0.f) || total <= p.list_len || pinned) break;  // uniform
+#pragma unroll 1
+    for (int shift = 8; shift >= 0; shift -= 8)
+      radix_pass_regs(sh, sh.hist[0], false, shift, key, prefix, mask, need, phantom);
+  }
   if (!(band == band && total <= p.list_len)) {  // uniform
     if (!(band == 0.f)) {
-      exact_scores(p, sh, (n + 15) >> 4, [&](int b, int c) { return min(c0 + b * 16 + c, p.S - 1); },
-                   [&](int b, int c, float v) {
-                     if (b * 16 + c < n) chunk[b * 16 + c] = v;
-                   });
+      int taken;
+      const bool safe = band == band;
+      store_row_pieces(p, sh, rc);
+      const int n_open = list_open(sh, n, key, safe ? lo : 0u, safe ? order_key(key_value(prefix) + band) : ~0u, taken);
+      exact_scores_many(p, sh, n_open, [&](int i) { return c0 + (int)sh.open[i]; },
+                        [&](int i, float v) { chunk[sh.open[i]] = v; });
       load_keys(chunk, n, key);
       to_keys(n, key);
+      keep_open(sh, key);
+      phantom = KEYS - n_open - taken;
     }
-    mark_exact(p, sh, n, key, KEYS - n);
+    mark_exact(p, sh, n, key, phantom);
     total = rank_marks<KEYS>(sh, n);
+    if (!(band == 0.f)) {  // the taken keep their estimates
+      load_keys(chunk, n, key);
+      to_keys(n, key);
+      __syncthreads();  // every wave's keys have arrived: the list may take their place
+    }
   }
   write_list(p, sh, n, c0, key, total, chunk);
 }
@@ -1226,34 +1432,30 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_merge_kernel(Indexe
   int need;
   find_bin(p, sh, key, 0, prefix, mask, need);  // (empty entries are the lowest keys)
   const float band = sh.band;
-  mark_taken(sh, KEYS, key, max(order_key(key_value(prefix) - band), 1u),
-             order_key(key_value(prefix | 0xffffu) + band), prefix | 0xffffu);
-  store_row_pieces(p, sh, rc);
-  __syncthreads();
-  const int n_open = sh.n_cand;
+  uint32_t top;
+  int n_open = mark_open(p, sh, rc, KEYS, key, 0, band, prefix, top, mask, need);
   if (band == band && n_open <= kMaxOpen) {  // uniform
-    exact_scores(p, sh, (n_open + 15) >> 4,
-                 [&](int b, int c) { return position((int)sh.cand[min(b * 16 + c, n_open - 1)].y); },
-                 [&](int b, int c, float v) {
-                   if (b * 16 + c < n_open) sh.cand[b * 16 + c].x = max(order_key(v), 1u);
-                 });
+    score_listed(p, sh, n_open, position);
     rank_open(sh, n_open, need + sh.n_above);
     write_marked<KEYS>(p, sh, t, KEYS, out, position);
     return;
   }
   __syncthreads();  // every wave has read n_cand: mark_exact clears it
-  // every listed position's exact score, then the selection from those
+  int phantom = 0;
   if (!(band == 0.f)) {
+    int taken;
     uint32_t *keys = (uint32_t *)row;
-    exact_scores(p, sh, places >> 4,
-                 [&](int b, int c) { return keys[entry(b * 16 + c)] != 0 ? position(b * 16 + c) : 0; },
-                 [&](int b, int c, float v) {
-                   uint32_t *k = keys + entry(b * 16 + c);
-                   if (*k != 0) *k = max(order_key(v), 1u);
-                 });
+    const bool safe = band == band;  // else every listed position is open
+    const uint32_t lo = safe ? max(order_key(key_value(prefix) - band), 1u) : 1u;
+    const uint32_t hi = safe ? order_key(key_value(top) + band) : ~0u;
+    n_open = list_open(sh, KEYS, key, lo, hi, taken);
+    exact_scores_many(p, sh, n_open, [&](int i) { return position((int)sh.open[i]); },
+                      [&](int i, float v) { keys[entry((int)sh.open[i])] = max(order_key(v), 1u); });
     load_lists();
+    keep_open(sh, key);
+    phantom = KEYS - n_open - taken;
   }
-  mark_exact(p, sh, KEYS, key, 0);
+  mark_exact(p, sh, KEYS, key, phantom);
   write_marked<KEYS>(p, sh, t, KEYS, out, position);
 }
 
