@@ -175,10 +175,11 @@ __global__ __launch_bounds__(kEstWaves * 64, SRC == kPrepared ? 2 : 1) void dsa_
             u32x4, __builtin_amdgcn_raw_buffer_load_b128(krs, kvo + 64 * j, blk * stride, 0));
     }
   };
-  // the scale of the lane's position of the pair starting at blk: block g >> 1
+  // 2^18 c_s of the lane's position of the pair starting at blk: block g >> 1
   auto fetch_cs = [&](int blk) {
-    const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(srs, ((g >> 1) * 16 + c) * 4, blk * 64, 0);
-    return __uint_as_float(v) * (SRC == kFlat ? 1.0f : 0x1p18f);
+    const float v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srs, ((g >> 1) * 16 + c) * 4, blk * 64, 0));
+    // (c_s, which the exact score and the bound take, is rounded where it is subnormal)
+    return (SRC == kFlat ? v * 0x1p-18f : v) * 0x1p18f;
   };
   // What dsa_idx_prep_kernel writes, of block blk (of the caller's K)
   auto prepare = [&](int blk, Raw &r) {

@@ -752,6 +752,24 @@ def test_crowded_rows_cost_about_what_ordinary_ones_do():
     assert slow < 3 * fast, times
 
 
+@pytest.mark.parametrize("T", [4, 9])  # K prepared by the estimate kernel, and before it
+@pytest.mark.parametrize("S", [3000, 40000])
+def test_selection_without_scores_of_subnormal_scales(T, S):
+    """c_s = fl32(k_scale * 2^-18) is 0 or a few units of the smallest subnormal:
+    every score is 0 and the first positions win, or scores differ only by
+    that rounding."""
+    d = workloads.indexer_inputs(T=T, Hi=32, S=S, seed=S + T)
+    d["causal_limit"] = torch.full((T,), S - 1, dtype=torch.int32)
+    scale = d["k_scale"]
+    for name, k_scale in (("all zero", torch.full((S,), 1e-41)), ("spread", scale * 1e-41),
+                          ("rounded", scale * 2.0 ** -130), ("among others", torch.where(scale > 1.5, scale, 1e-41))):
+        print(f"subnormal scales: {name} T={T} S={S}", flush=True)
+        got, want = _select_both(dict(d, k_scale=k_scale.float()), 300)
+        assert np.array_equal(got, want), name
+        if name in ("all zero", "spread"):
+            assert np.array_equal(got, np.tile(np.arange(300, dtype=np.int32), (T, 1))), name
+
+
 def test_selection_without_scores_after_nan_filled_lds():
     for S in (20000, 45000):
         d = _full_range(workloads.indexer_inputs(T=5, Hi=64, S=S, seed=77), torch.Generator().manual_seed(78))
