@@ -230,9 +230,9 @@ int dsa_attn_merge(const dsa_attn_merge_args *args, void *stream);
  * workspace (dsa_indexer_workspace_bytes, 256-byte aligned) holds the MFMA
  * operand pieces of k and, unless scores_out is given, the scores or their
  * estimates (a selection whose scores are not returned computes exact scores
- * only where estimates, proven to lie within a bound of them, leave the
- * choice open: the same sets); a call whose workspace size is 0 may pass
- * NULL.
+ * only where estimates leave the choice open, by a bound on their distance
+ * five times what the matrix unit's fp32 sums were measured to lose: the same
+ * sets); a call whose workspace size is 0 may pass NULL.
  */
 typedef struct dsa_indexer_args {
   const uint8_t *q_idx;

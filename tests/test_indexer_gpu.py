@@ -7,6 +7,7 @@ going to the lower position.  Reference: solution/triton/indexer_kernel.py
 :4-343 (score structure :185-275, intended selection :289-343) and the
 BASELINE indexer workload (config 5).
 """
+import ctypes
 import math
 import os
 
@@ -768,6 +769,88 @@ def test_selection_without_scores_of_subnormal_scales(T, S):
         assert np.array_equal(got, want), name
         if name in ("all zero", "spread"):
             assert np.array_equal(got, np.tile(np.arange(300, dtype=np.int32), (T, 1))), name
+
+
+def _estimates(q, k, k_scale, w, topk):
+    """What a call without scores leaves in its workspace: a row's estimates (its
+    last T x S floats), except where exact scores took their place, which only
+    rows with more than 512 positions close to the k-th have."""
+    q, k, k_scale, w = (x.to(DEV).contiguous() for x in (q, k, k_scale, w))
+    T, Hi, _ = q.shape
+    S = k.shape[0]
+    lim = torch.full((T,), S - 1, dtype=torch.int32, device=DEV)
+    lib = _lib.load()
+    n = lib.dsa_indexer_workspace_bytes(T, Hi, 128, S)
+    ws = torch.zeros(n, dtype=torch.uint8, device=DEV)
+    out = torch.empty((T, topk), dtype=torch.int32, device=DEV)
+    a = _lib.IndexerArgs()
+    a.q_idx, a.k_idx, a.k_scale, a.weights = q.data_ptr(), k.data_ptr(), k_scale.data_ptr(), w.data_ptr()
+    a.causal_limit, a.out = lim.data_ptr(), out.data_ptr()
+    a.num_tokens, a.num_heads, a.head_dim, a.num_positions, a.topk = T, Hi, 128, S, topk
+    a.workspace, a.workspace_bytes = ws.data_ptr(), n
+    _lib.check("dsa_indexer_topk",
+               lib.dsa_indexer_topk(ctypes.byref(a), torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    first = n - (T * S * 4 + 255) // 256 * 256
+    return ws[first:first + T * S * 4].view(torch.float32).view(T, S).double().cpu()
+
+
+@pytest.mark.parametrize("T", [8, 16])  # K prepared by the estimate kernel, and before it
+@pytest.mark.parametrize("at", [0, 7, 8, 40, 127])
+def test_estimated_dots_of_directed_codes_stay_within_their_share_of_the_bound(T, at):
+    """One large product at dim `at` beside 127 of every magnitude and sign: the
+    sums' losses add up.  One head has weight 1, so an estimate is a dot.  16
+    sums truncated to 24 bits lose at most 16 x 2^-23 of |q| |k|; the bound
+    allows 2^-17."""
+    levels = [2.0 ** e * (1 + m / 8) for e in range(-9, 9) for m in range(8) if 2.0 ** e * (1 + m / 8) <= 448]
+    rows = []
+    for big in (448.0, 416.0, 256.0, 288.0):
+        for v in levels:
+            for pattern in range(3):
+                r = torch.full((128,), v if pattern != 1 else -v)
+                if pattern == 2:
+                    r[1::2] *= -1
+                r[at] = big
+                rows.append(r)
+    top = torch.zeros(20, 128)      # the selected rows lie far above: the others are not near the k-th
+    top[:, at] = 448.0
+    k = workloads.e4m3(torch.cat([top, torch.stack(rows)]))
+    k_scale = torch.ones(len(k))
+    k_scale[:20] = 8.0
+    w = torch.zeros(T, 16)
+    w[torch.arange(T), torch.arange(T)] = 1.0
+    worst = 0.0
+    for small in (2.0 ** -9, 2.0 ** -6, 2.0 ** -4, 0.25, 1.0, 4.0):
+        q = torch.zeros(T, 16, 128)
+        for t in range(T):
+            q[t, t] = small * (1 + (t % 8) / 8)
+            q[t, t, at] = (448.0, 416.0, 384.0, 320.0, 256.0, 288.0, 352.0, 240.0)[t % 8]
+        q = workloads.e4m3(q)
+        est = _estimates(q, k, k_scale, w, 10)[:, 20:]
+        qv = q.view(torch.float8_e4m3fn).double()[torch.arange(T), torch.arange(T)]
+        kv = k.view(torch.float8_e4m3fn).double()[20:]
+        err = (est - (qv @ kv.t()).clamp_min(0.0)).abs() / (qv.norm(dim=1)[:, None] * kv.norm(dim=1)[None])
+        worst = max(worst, float(err.max()))
+    print(f"largest loss at dim {at}, T={T}: 2^{math.log2(worst):.2f}", flush=True)
+    assert worst <= 16 * 2.0 ** -23
+
+
+@pytest.mark.parametrize("full_range", [False, True])
+def test_estimates_of_ordinary_rows_stay_within_the_bound(full_range):
+    T, Hi, S = 12, 64, 5000
+    d = workloads.indexer_inputs(T=T, Hi=Hi, S=S, seed=404)
+    if full_range:
+        d = _full_range(d, torch.Generator().manual_seed(405))
+    d["causal_limit"] = torch.full((T,), S - 1, dtype=torch.int32)
+    est = _estimates(d["q_idx"], d["k_idx"], d["k_scale"], d["weights"], 300)
+    g = workloads.to_device(d, DEV)
+    _, sc = run_indexer_and_topk(g["q_idx"], g["k_idx"], g["k_scale"], g["weights"], g["causal_limit"], 300,
+                                 return_scores=True)
+    torch.cuda.synchronize()
+    qn = d["q_idx"].view(torch.float8_e4m3fn).double().norm(dim=2)
+    kn = (d["k_idx"].view(torch.float8_e4m3fn).double().norm(dim=1) * d["k_scale"].double().abs()).max()
+    bound = 1.328125 * 2.0 ** -17 * (d["weights"].double().abs() * qn).sum(1) * kn
+    assert ((est - sc.double().cpu()).abs() <= bound[:, None]).all()
 
 
 def test_selection_without_scores_after_nan_filled_lds():
