@@ -771,6 +771,79 @@ def test_selection_without_scores_of_subnormal_scales(T, S):
             assert np.array_equal(got, np.tile(np.arange(300, dtype=np.int32), (T, 1))), name
 
 
+HARD = ["many equal rows", "nearly equal rows", "outlier rows", "outlier scales", "zero rows", "wide exponents",
+        "zero weights", "zero queries", "tiny weights", "huge weights", "weights not finite", "scales not finite",
+        "NaN codes"]
+
+
+# K prepared on the estimate kernel's way (up to 8 tokens) and by its own kernel;
+# rows in registers and in chunks; cache pages that end inside a 16-position
+# block, or lie on one
+@pytest.mark.parametrize("T,S,page", [(4, 7001, 20), (9, 7001, 64), (8, 40003, 64), (9, 40003, 12)])
+@pytest.mark.parametrize("kind", HARD + CROWDED)
+def test_selection_without_scores_over_every_k_source(kind, T, S, page):
+    """Flat, paged and planes calls take the positions of the call that returns
+    scores, for hard and crowded rows, with some pages unmapped (-1, ids past
+    the cache): their positions are zero rows of scale 0."""
+    from dsa_amd import prepare_k, prepare_k_paged, run_indexer_and_topk_paged
+    d = (_hard if kind in HARD else _crowded)(kind, T, 64 if T == 9 else 32, S)
+    gen = torch.Generator().manual_seed(S + page)
+    n_pages = -(-S // page)
+    page_of = torch.randperm(n_pages, generator=gen).to(torch.int32)
+    pos = torch.arange(S)
+    codes = torch.zeros(n_pages, page, 128, dtype=torch.uint8)
+    scale = torch.zeros(n_pages, page)
+    codes[page_of[pos // page].long(), pos % page] = d["k_idx"].view(torch.uint8)
+    scale[page_of[pos // page].long(), pos % page] = d["k_scale"].float()
+    cache = torch.cat([codes.view(n_pages, -1), scale.view(torch.uint8).view(n_pages, -1)], dim=1).contiguous()
+    unmapped = [1, n_pages // 2, n_pages - 1]
+    for pg, bad in zip(unmapped, (-1, n_pages, 2 ** 31 - 1)):
+        page_of[pg] = bad
+    gone = torch.isin(pos // page, torch.tensor(unmapped))
+    k, ks = d["k_idx"].view(torch.uint8).clone(), d["k_scale"].float().clone()
+    k[gone], ks[gone] = 0, 0.0
+    g = workloads.to_device(dict(d, k_idx=k, k_scale=ks), DEV)
+    cache, pages = cache.to(DEV).view(n_pages, -1), page_of.to(DEV)
+    rest = (g["weights"], g["causal_limit"])
+    flat_planes = prepare_k(g["k_idx"], g["k_scale"])
+    paged_planes = prepare_k_paged(cache, pages, S)
+    for topk in (300, 2048):
+        print(f"K sources: {kind} T={T} S={S} page={page} k={topk}", flush=True)
+        want, _ = run_indexer_and_topk(g["q_idx"], g["k_idx"], g["k_scale"], *rest, topk, return_scores=True)
+        got = {"flat": run_indexer_and_topk(g["q_idx"], g["k_idx"], g["k_scale"], *rest, topk),
+               "paged": run_indexer_and_topk_paged(g["q_idx"], cache, pages, S, *rest, topk),
+               "planes of flat": run_indexer_and_topk(g["q_idx"], None, None, *rest, topk, k_planes=flat_planes),
+               "planes of paged": run_indexer_and_topk(g["q_idx"], None, None, *rest, topk, k_planes=paged_planes)}
+        torch.cuda.synchronize()
+        for name, x in got.items():
+            assert torch.equal(x, want), f"{kind}, {name}, k={topk}"
+
+
+@pytest.mark.parametrize("Hi", [16, 32, 48, 64])
+@pytest.mark.parametrize("T", [1, 2, 5, 8])
+def test_paged_selection_without_scores_matches_oracle(T, Hi):
+    """The estimate kernel reading a paged cache itself (up to 8 tokens), every
+    head count, tokens below and at its pairs and fours, limits inside a page."""
+    from dsa_amd import run_indexer_and_topk_paged
+    S, ps, topk = 2500 + 100 * T, 64, 600
+    d = _full_range(workloads.indexer_inputs(T=T, Hi=Hi, S=S, seed=Hi + T), torch.Generator().manual_seed(Hi * 10 + T))
+    lim = torch.randint(topk - 5, S, (T,), generator=torch.Generator().manual_seed(T))
+    d["causal_limit"] = lim.to(torch.int32)
+    n_pages = -(-S // ps)
+    page_of = torch.randperm(n_pages + 3, generator=torch.Generator().manual_seed(S))[:n_pages].to(torch.int32)
+    pos = torch.arange(S)
+    slots = (page_of[pos // ps].long() * ps + pos % ps).numpy()
+    cache = oracle.pack_k_cache(np.zeros((n_pages + 3, ps * 132), np.uint8), d["k_idx"].view(torch.uint8).numpy(),
+                                d["k_scale"].numpy(), slots, ps)
+    g = workloads.to_device(d, DEV)
+    print(f"paged selection T={T} Hi={Hi} S={S}", flush=True)
+    got = run_indexer_and_topk_paged(g["q_idx"], torch.from_numpy(cache).to(DEV), page_of.to(DEV), S, g["weights"],
+                                     g["causal_limit"], topk)
+    torch.cuda.synchronize()
+    ref, _ = _oracle(d, topk)
+    assert np.array_equal(np.sort(got.cpu().numpy(), axis=1), np.sort(ref, axis=1))
+
+
 def _estimates(q, k, k_scale, w, topk):
     """What a call without scores leaves in its workspace: a row's estimates (its
     last T x S floats), except where exact scores took their place, which only
