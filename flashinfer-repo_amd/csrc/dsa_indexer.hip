@@ -75,10 +75,10 @@ constexpr int kTargetScoreWaves = 2048;   // two waves per SIMD on 256 CUs
 constexpr int kMinBlocksPerWave = 8;
 
 // K blocks k_block0 .. k_block0 + k_blocks - 1 (16 positions each): c_s of
-// every position, the k_max word of every block (largest |x| and largest
-// |c_s| * |k_s|) and, by WHAT, the codes row by row without NaN codes and the
-// piece planes laid out as MFMA B operands in lane order (one 1 KB chunk per
-// plane and 64-wide k-step): planes p0 and p1, then (kPrepDiff) a plane of p2 if
+// every position, the k_max word of every block (largest |x| and, but for
+// kPrepDiff, largest |c_s| * |k_s|) and, by WHAT, the codes row by row without
+// NaN codes and the piece planes laid out as MFMA B operands in lane order (one
+// 1 KB chunk per plane and 64-wide k-step): planes p0 and p1, then (kPrepDiff) a plane of p2 if
 // the block holds a value of magnitude >= 32, else of p0 - p1.  One wave per
 // block; lane l = 16*g + c holds position 16*block + c at dims 64*ks + 16*g for
 // k-steps ks = 0, 1, so every plane store of the wave is one contiguous 1 KB
@@ -119,16 +119,19 @@ __global__ __launch_bounds__(kPrepThreads) void dsa_idx_prep_kernel(IndexerParam
   const uint32_t w[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[1].x, raw[1].y, raw[1].z, raw[1].w};
   const int bmax = magnitude_bound(wave_top_code(w));
   uint32_t v[8];
-  float n2 = 0.f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) v[i] = drop_nan(w[i]);
+  uint32_t nb = 0;
+  if constexpr (WHAT != kPrepDiff) {  // (exact scores need no norms)
+    float n2 = 0.f;
 #pragma unroll
-  for (int i = 0; i < 8; i += 2) n2 += sum_squares8(v[i], v[i + 1]);
-  n2 += __shfl_xor(n2, 16);  // the position's four lanes
-  n2 += __shfl_xor(n2, 32);
-  uint32_t nb = position_norm_bits(cs, n2);
+    for (int i = 0; i < 8; i += 2) n2 += sum_squares8(v[i], v[i + 1]);
+    n2 += __shfl_xor(n2, 16);  // the position's four lanes
+    n2 += __shfl_xor(n2, 32);
+    nb = position_norm_bits(cs, n2);
 #pragma unroll
-  for (int o = 8; o > 0; o >>= 1) nb = max(nb, (uint32_t)__shfl_xor((int)nb, o));
+    for (int o = 8; o > 0; o >>= 1) nb = max(nb, (uint32_t)__shfl_xor((int)nb, o));
+  }
   if (lane == 0) p.k_max[blk] = (int32_t)((uint32_t)bmax | (nb << kMaxXBits));
 
   // non-temporal stores: the planes are read by the next kernel, and stores
