@@ -2091,14 +2091,14 @@ hipError_t launch_attention_partial(const AttnParams &p, hipStream_t stream) {
     // of the eight-wave layout, each gathering the chunk's keys for about 0.6
     // of its time -- finish sooner while that grid fits the CUs in one round
     // (H=128, top-k 2048: T=16 32 us against 42 us for eight-wave workgroups
-    // and 16 splits, T=32 43 against 53 us), and in three rounds where the
-    // eight-wave grid takes two (T=86 130 against 144 us, T=100 136 against
-    // 147; T=125 at top-k 1024 109 both).  With one or two chunks the shared
-    // gathers count for more: T=190, top-k 512 97 against 94 us, 300 tokens of
-    // a prompt 52 against 45; in two rounds against one T=128 131 against 121.
-    // The same bits either way.
-    const int64_t blocks = (int64_t)p.T * p.num_splits * (groups / 4);
-    if (blocks <= kNumCU || (p.num_splits >= 3 && blocks > 2 * kNumCU && blocks <= 3 * kNumCU))
+    // and 16 splits, T=32 43 against 53 us).  Past that the eight-wave
+    // workgroups' shared gathers win, or their other team hides the rescaling
+    // that scores of many sizes call for: where the four-wave grid takes three
+    // rounds to their two it gains on cache rows of one size (T=70 107 against
+    // 118 us, T=100 130 against 144) and loses with one row in twenty eight
+    // times as large (132 against 121, 165 against 148).  The same bits either
+    // way.
+    if ((int64_t)p.T * p.num_splits * (groups / 4) <= kNumCU)
       return launch_ring<4, 1>(p, groups / 4, stream);
     return launch_ring<8, 1>(p, hb, stream);  // one wave per head group
   }
