@@ -137,11 +137,21 @@ __global__ __launch_bounds__(kPrepThreads) void dsa_idx_prep_kernel(IndexerParam
   // non-temporal stores: the planes are read by the next kernel, and stores
   // kept in L2 cost a write-back at the kernel's end (measured: 1.6 us of 10.8)
   if constexpr (WHAT != kPrepDiff) {
-    uint8_t *codes = p.k_codes + (int64_t)blk * p.k_code_stride + c * kIdxDim + g * 16;
+    // lanes c and c ^ 8 of a row of 16 exchange halves, so that a store covers
+    // eight whole rows (1 KB) and not one half of sixteen: planes of 524288
+    // positions 46.3 -> 42.7 us
+    const bool low = c < 8;
+    uint8_t *codes = p.k_codes + (int64_t)blk * p.k_code_stride + (c & 7) * kIdxDim + (low ? 0 : 64) + g * 16;
+    u32x4 top, bottom;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-      __builtin_nontemporal_store(u32x4{v[4 * ks], v[4 * ks + 1], v[4 * ks + 2], v[4 * ks + 3]},
-                                  (u32x4 *)(codes + 64 * ks));
+    for (int d = 0; d < 4; ++d) {
+      const uint32_t other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(low ? v[4 + d] : v[d]), 0x128,  // row_ror:8
+                                                                     0xf, 0xf, false);
+      top[d] = low ? v[d] : other;
+      bottom[d] = low ? other : v[4 + d];
+    }
+    __builtin_nontemporal_store(top, (u32x4 *)codes);
+    __builtin_nontemporal_store(bottom, (u32x4 *)(codes + 8 * kIdxDim));
   }
   if constexpr (WHAT != kPrepCodes) {
     uint32_t pw[32];
