@@ -242,7 +242,10 @@ int prepare_attn(const char *fn, const dsa_attn_args *a, bool partial_only, dsa:
   p->H = (int32_t)a->num_heads;
   p->K = (int32_t)a->topk;
   p->page_size = (int32_t)a->page_size;
-  p->num_slots = a->num_pages * a->page_size;
+  // slot ids are int32 and the kernels compare them as 32-bit numbers: of a cache
+  // of more slots (a view whose pages repeat) every id from 0 on is one
+  constexpr int64_t kAllSlots = int64_t(1) << 31;
+  p->num_slots = a->num_pages > kAllSlots / a->page_size ? kAllSlots : a->num_pages * a->page_size;
   {
     int sh = 0;
     while ((int64_t(1) << sh) < a->page_size) ++sh;

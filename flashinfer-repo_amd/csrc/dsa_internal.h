@@ -36,7 +36,7 @@ struct AttnParams {
   float *lse;  // element strides
   int64_t lse_st, lse_sh;
   int32_t T, H, K, page_size;
-  int64_t num_slots;
+  int64_t num_slots;  // at most 2^31
   // slot / page_size = (slot * ps_magic) >> (31 + ps_shift) for every slot
   // below 2^31 (round-up reciprocal: ps_shift = ceil(log2 page_size),
   // ps_magic = floor(2^(31 + ps_shift) / page_size) + 1 < 2^32)

@@ -806,3 +806,26 @@ def test_outlier_rows_cost_a_split_batch_of_all_heads_little():
         times.append(best)
     print("ordinary rows %.1f us, outlier rows %.1f us" % tuple(times), flush=True)
     assert times[1] < 1.15 * times[0], times
+
+
+@pytest.mark.parametrize("H,T", [(16, 3), (32, 40), (64, 9), (128, 9)])
+def test_cache_views_of_more_slots_than_int32_counts(H, T):
+    """A cache view whose one page repeats 2^27 times has 2^33 slots: every id from
+    0 to 2^31 - 1 is one of them, negative ids are padding."""
+    page, K = 64, 2048
+    g = torch.Generator().manual_seed(H)
+    d = workloads.attention_inputs(T, H, K, 1, page, seed=H)
+    d.pop("gen")
+    idx = torch.randint(0, 2 ** 31 - 1, (T, K), generator=g, dtype=torch.int64)
+    idx[:, 0], idx[:, 1] = 2 ** 31 - 1, 0
+    idx[:, 5::9] = -1
+    idx[:, 6::11] = -(2 ** 31)
+    d.update(sparse_indices=torch.where(idx < 0, idx, idx % page).clamp_min(-1).to(torch.int32),
+             sm_scale=workloads.SM_SCALE)
+    ref = _oracle(d)
+    dev = workloads.to_device({k: d[k] for k in ("q_nope", "q_pe", "ckv_cache", "kpe_cache")}, DEV)
+    print(f"2^33 slots H={H} T={T}", flush=True)
+    out, lse = kernel(dev["q_nope"], dev["q_pe"], dev["ckv_cache"].expand(2 ** 27, page, 512),
+                      dev["kpe_cache"].expand(2 ** 27, page, 64), idx.to(torch.int32).to(DEV), d["sm_scale"])
+    torch.cuda.synchronize()
+    _assert_parity(out.cpu(), lse.cpu(), *ref, f"2^33 slots H={H}")
