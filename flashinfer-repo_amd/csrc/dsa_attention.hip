@@ -567,7 +567,10 @@ __device__ __forceinline__ void item_issue(const TileAddr &a, ItemRegs &r) {
 // stream are written out: left to itself the compiler places the result of
 // each where it likes and copies accumulators between registers (64 heads,
 // 300 tokens, top-k 2048: 213 us with builtins, 185 so).  scores_settled and
-// accumulators_settled stand for the hazards it then does not know of.
+// accumulators_settled stand for the hazards it then does not know of.  It
+// keeps no wait states between a move and an operand of these MFMAs either
+// (two are needed), nor between an LDS read and a move of its result before the
+// wait: tests/test_asm_hazards.py looks for both in the compiled code.
 template <int N, bool FIRST>
 __device__ __forceinline__ void item_qk(const u32x4 (&k)[2], const bf16x8 &q, f32x4 (&s)[2]) {
   if constexpr (FIRST)
