@@ -489,15 +489,17 @@ extern "C" __device__ int amdgcn_writelane(int value, int lane, int old) __asm("
 // many; more are selected from by radix passes over their exact keys.
 constexpr int kMaxSurvivors = 256;
 constexpr int kMaxOpen = 512;
-// From estimates: with more open positions than kMaxBinOpen two more passes pin
-// the k-th estimate itself, so that only those within twice the bound of it stay
-// open, not those of its whole 16-bit bin (2^-7 of its value: where q and K share
-// a component, hundreds to thousands).  64 rows of 32768 positions with a shared
-// component four times the noise: 1393 us when a crowded bin was scored whole,
-// 60 now; ordinary rows have about 100 open and stay at 53.  (The passes cost
-// less than scoring 128 more: 4 rows of 8000, shared component, 22.6 us with a
-// limit of 256, 20.8 with 128.)
+// From estimates: the open positions are first those of the k-th estimate's
+// 16-bit bin (2^-7 of its value: about 100 of an ordinary row of 32768, hundreds
+// to thousands where the weights have one sign or q and K share a component).
+// With more than kMaxBinOpen they are narrowed to those within twice the bound of
+// the k-th estimate itself, a handful: by ranking the list up to kMaxNarrowed
+// (narrow_open; rows past 8192 positions only: the shorter ones' kernel takes
+// 0.2 us longer with it whatever the row), past that by two more radix passes,
+// which cost 4 us.  (64 rows of 32768 positions with a shared component four times
+// the noise took 1393 us when a crowded bin was scored whole, 55 now.)
 constexpr int kMaxBinOpen = 128;
+constexpr int kMaxNarrowed = 256;
 
 // Shared state of one top-k workgroup (KEYS = positions it holds).  One
 // space serves the radix histograms, then the row's q pieces, then the
@@ -531,6 +533,8 @@ struct TopkShared {
   int2 scan[kTopkThreads / 64 + 1];
   uint32_t prefix, mask;
   int need, n_cand, n_above;  // n_above: open keys above the k-th largest key's bin
+  uint32_t kth;               // narrow_open: the k-th key, and how many listed keys
+  int n_sure, n_left;         // are taken for sure and how many stay open
 };
 
 // Rows with at most topk candidates: every candidate, then -1.
@@ -823,7 +827,10 @@ __device__ __forceinline__ void clear_counts(Shared &sh) {
   static_assert(2 * kHistCopies * kHistPitch % 4 == 0, "zeroed 16 bytes at a time");
   for (int i = threadIdx.x; i < 2 * kHistCopies * kHistPitch / 4; i += kTopkThreads)
     ((u32x4 *)&sh.hist[0][0])[i] = u32x4{0u, 0u, 0u, 0u};
-  if (threadIdx.x == 0) sh.n_cand = sh.n_above = 0;
+  if (threadIdx.x == 0) {
+    sh.n_cand = sh.n_above = sh.n_sure = sh.n_left = 0;
+    sh.kth = 0;
+  }
 }
 
 // Scores to order keys.  Adding +0.0 turns -0.0 into +0.0; the key orders the
@@ -860,7 +867,11 @@ template <int EPT, typename Shared>
 __device__ __forceinline__ void mark_taken(Shared &sh, int n, const uint32_t (&key)[EPT], uint32_t lo,
                                            uint32_t hi, uint32_t top) {
   constexpr int kWaves = kTopkThreads / 64;
-  const int tid = threadIdx.x, lane = tid & 63;
+  int tid = threadIdx.x;
+  // many keys' positions are made here, not kept from to_keys on (32 registers:
+  // 64 rows of 32768 49.6 -> 47.2 us)
+  if constexpr (EPT > 8) asm volatile("" : "+v"(tid));
+  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // known uniform: scalar masks
   uint32_t *bits32 = (uint32_t *)sh.bits;  // word w: positions 32w .. 32w+31
   // The selection as a position bitmap, built from ballots of the registers
@@ -1100,12 +1111,54 @@ __device__ __forceinline__ void store_row_pieces(const IndexerParams &p, Shared 
     store_pieces8(sh.lut, sh.qp + r.hb * (6 * kChunk), r.row, (threadIdx.x & 15) * 8, r.codes);
 }
 
+// Narrows the list (at most kMaxNarrowed) to the keys within band of the k-th
+// key, which is the need-th largest listed one; the keys above are marked, and
+// `need` falls by as many.  Returns how many are left.  Four lanes per key, as in
+// rank_open.  Once per workgroup.
+template <typename Shared>
+__device__ __forceinline__ int narrow_open(Shared &sh, int n_open, float band, int &need) {
+  static_assert(kMaxNarrowed <= kTopkThreads / 4, "one key per four lanes");
+  const int i = threadIdx.x >> 2, q = threadIdx.x & 3, lane = threadIdx.x & 63;
+  const bool mine = q == 0 && i < n_open;
+  const uint2 me = sh.cand[min(i, n_open - 1)];
+  int reach = 0;  // listed keys of at least mine
+  if (i < ((n_open + 15) & ~15)) {  // whole waves
+    for (int j0 = q; j0 < n_open; j0 += 16) {
+      uint32_t c[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) c[u] = sh.cand[min(j0 + 4 * u, kMaxOpen - 1)].x;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) reach += j0 + 4 * u < n_open && c[u] >= me.x;
+    }
+    reach += __builtin_amdgcn_update_dpp(0, reach, 0xb1, 0xf, 0xf, false);  // quad_perm [1,0,3,2]
+    reach += __builtin_amdgcn_update_dpp(0, reach, 0x4e, 0xf, 0xf, false);  // quad_perm [2,3,0,1]
+  }
+  if (mine && reach >= need) atomicMax(&sh.kth, me.x);
+  __syncthreads();  // (and every wave has read the list)
+  const float kth = key_value(sh.kth);
+  const uint32_t lo = max(order_key(kth - band), 1u), hi = order_key(kth + band);
+  const bool sure = mine && me.x > hi, open = mine && me.x >= lo && me.x <= hi;
+  if (sure) atomicOr((uint32_t *)sh.bits + (me.y >> 5), 1u << (me.y & 31));
+  const uint64_t sb = __ballot(sure), ob = __ballot(open);
+  int o = 0;
+  if (lane == 0) {
+    if (sb != 0) atomicAdd(&sh.n_sure, __popcll(sb));
+    if (ob != 0) o = atomicAdd(&sh.n_left, __popcll(ob));
+  }
+  o = __builtin_amdgcn_readfirstlane(o) +
+      __builtin_amdgcn_mbcnt_hi((uint32_t)(ob >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ob, 0));
+  if (open) sh.cand[o] = me;
+  __syncthreads();
+  need -= sh.n_sure;
+  return sh.n_left;
+}
+
 // Marks the keys that are taken for sure and lists the open ones: those within
 // band of the k-th key's bin [prefix, top], or, where they are many (see
 // kMaxBinOpen) and the band is a safe bound, within band of the k-th key
-// itself, which two more passes give (prefix == top then).  Returns how many
-// are open; `need` of the keys up to top, and the n_above open ones above it,
-// are among the k largest.  With the row's q pieces in the histograms' place.
+// itself (prefix == top where two more passes gave it).  Returns how many are
+// open, of which `need` are among the k largest.  With the row's q pieces in
+// the histograms' place.
 template <int EPT, typename Shared>
 __device__ __forceinline__ int mark_open(const IndexerParams &p, Shared &sh, const RowCodes &rc, int n,
                                          const uint32_t (&key)[EPT], int phantom, float band, uint32_t &prefix,
@@ -1117,8 +1170,15 @@ __device__ __forceinline__ int mark_open(const IndexerParams &p, Shared &sh, con
     store_row_pieces(p, sh, rc);
     __syncthreads();
     const int n_open = sh.n_cand;
-    if (!(band > 0.f) || n_open <= kMaxBinOpen || top == prefix) return n_open;  // uniform
-    __syncthreads();  // every wave has read n_cand
+    const int above = sh.n_above;
+    constexpr int kNoPasses = EPT > 8 ? kMaxNarrowed : kMaxBinOpen;
+    if (!(band > 0.f) || n_open <= kNoPasses || top == prefix) {  // uniform
+      need += above;  // (the keys above the bin, or the k-th, that are open are not taken for sure)
+      if constexpr (EPT > 8)
+        if (band > 0.f && n_open > kMaxBinOpen && top != prefix) return narrow_open(sh, n_open, band, need);
+      return n_open;
+    }
+    __syncthreads();  // every wave has read the counts
     if (threadIdx.x == 0) sh.n_cand = sh.n_above = 0;
 #pragma unroll 1
     for (int shift = 8; shift >= 0; shift -= 8)
@@ -1251,8 +1311,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_estimates_kernel(In
   int n_open = mark_open(p, sh, rc, n, key, phantom, band, prefix, top, mask, need);
   if (band == band && n_open <= kMaxOpen) {  // uniform
     score_listed(p, sh, n_open, [](int i) { return i; });
-    // (the keys above the bin, or the k-th, that are open are not taken for sure)
-    rank_open(sh, n_open, need + sh.n_above);
+    rank_open(sh, n_open, need);
     write_marked<KEYS>(p, sh, t, n, out, [](int i) { return i; });
     return;
   }
@@ -1442,7 +1501,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_merge_kernel(Indexe
   int n_open = mark_open(p, sh, rc, KEYS, key, 0, band, prefix, top, mask, need);
   if (band == band && n_open <= kMaxOpen) {  // uniform
     score_listed(p, sh, n_open, position);
-    rank_open(sh, n_open, need + sh.n_above);
+    rank_open(sh, n_open, need);
     write_marked<KEYS>(p, sh, t, KEYS, out, position);
     return;
   }

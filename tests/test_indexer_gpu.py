@@ -725,6 +725,35 @@ def test_selection_without_scores_of_crowded_rows(kind, S, topk):
     assert np.array_equal(got, want), kind
 
 
+# a row in registers of each size, and in chunks and their lists
+@pytest.mark.parametrize("S", [8000, 16000, 32768, 40000])
+def test_selection_with_every_length_of_the_open_list(S):
+    """Lists of open positions at the lengths where the selection goes another
+    way: scored as they are up to 128, narrowed by ranking up to 256 (rows past
+    8192 positions), by two more radix passes past that.  The top-k is chosen by how many scores share
+    the 16-bit bin of the k-th."""
+    d = _crowded("shared component", 1, 64, S)
+    d["causal_limit"][:] = S - 1
+    g = workloads.to_device(d, DEV)
+    args = (g["q_idx"], g["k_idx"], g["k_scale"], g["weights"], g["causal_limit"])
+    scores = run_indexer_and_topk(*args, 1, return_scores=True)[1].cpu().numpy()[0]
+    desc = np.sort(scores)[::-1]
+    assert desc[0] > 0
+    bins, count = np.unique(desc.view(np.uint32) >> 16, return_counts=True)
+    size = dict(zip(bins.tolist(), count.tolist()))
+    share = np.array([size[b] for b in (desc.view(np.uint32) >> 16).tolist()])  # of the k-th score's bin
+    taken = 0
+    for lo, hi in ((1, 64), (65, 110), (135, 190), (190, 250), (262, 400), (400, 505), (520, 100000)):
+        at = np.nonzero((share[:9000] >= lo) & (share[:9000] <= hi) & (desc[:9000] > 0))[0]
+        for k in sorted({int(x) + 1 for x in (at[:1].tolist() + at[at.size // 2:at.size // 2 + 1].tolist() + at[-1:].tolist())}):
+            print(f"open list S={S} k={k} bin {share[k - 1]}", flush=True)
+            got = run_indexer_and_topk(*args, k).cpu().numpy()
+            want = run_indexer_and_topk(*args, k, return_scores=True)[0].cpu().numpy()
+            assert np.array_equal(got, want), (k, share[k - 1])
+            taken += 1
+    assert taken >= 12
+
+
 def test_crowded_rows_cost_about_what_ordinary_ones_do():
     """Scores that share a large mean put hundreds of positions into the k-th
     one's bin, few of them within the estimates' bound of it: 64 rows take
