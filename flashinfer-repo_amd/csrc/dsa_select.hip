@@ -1611,8 +1611,21 @@ bool estimates_apply(const IndexerParams &p) {
 
 // Few tokens: the estimate kernel is bound by latency and prepares K on its way
 // (a launch less: 3 tokens, 2500 positions, 32 heads 20.6 -> 16.1 us); from 9
-// tokens on several workgroups would prepare the same blocks.
-bool estimates_prepare_k(const IndexerParams &p) { return p.T <= kEstFusedTokens; }
+// tokens on several workgroups would prepare the same blocks.  With more than
+// one pair of tokens the waves of a workgroup already do, and a kernel that holds
+// the operands of many heads beside its preparation runs one wave per SIMD: where
+// that costs more than a launch, long rows are prepared first.  8 tokens of 64 heads over
+// 32768 positions: paged 40.5 -> 32.4 us, flat 35.5 -> 32.4; over 131071: 95.9 ->
+// 65.6, 79.7 -> 66.1; 4 tokens, paged, 32768: 35.1 -> 31.5.  Kept: flat, 2 tokens of
+// 64 heads over 131071 52 us against 58, 8 of 48 heads over 32768 29.6 against
+// 31.4; paged, 4 tokens of 32 heads over 65536 44.4 against 46.5.
+bool estimates_prepare_k(const IndexerParams &p) {
+  if (p.T > kEstFusedTokens) return false;
+  const int pairs = (p.T + 1) / 2;
+  const int64_t work = (int64_t)pairs * p.S;
+  if (p.k_cache != nullptr) return p.Hi > 32 ? work <= 32768 : pairs <= 2 || work <= 65536;
+  return p.Hi <= 48 || pairs <= 2 || work <= 65536;
+}
 
 hipError_t launch_estimates(const IndexerParams &pin, hipStream_t stream) {
   IndexerParams p = pin;

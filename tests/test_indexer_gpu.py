@@ -805,10 +805,10 @@ HARD = ["many equal rows", "nearly equal rows", "outlier rows", "outlier scales"
         "NaN codes"]
 
 
-# K prepared on the estimate kernel's way (up to 8 tokens) and by its own kernel;
-# rows in registers and in chunks; cache pages that end inside a 16-position
-# block, or lie on one
-@pytest.mark.parametrize("T,S,page", [(4, 7001, 20), (9, 7001, 64), (8, 40003, 64), (9, 40003, 12)])
+# K prepared on the estimate kernel's way (up to 8 tokens; a paged cache's long
+# rows up to 4) and by its own kernel; rows in registers and in chunks; cache
+# pages that end inside a 16-position block, or lie on one
+@pytest.mark.parametrize("T,S,page", [(4, 7001, 20), (9, 7001, 64), (4, 40003, 64), (8, 40003, 64), (9, 40003, 12)])
 @pytest.mark.parametrize("kind", HARD + CROWDED)
 def test_selection_without_scores_over_every_k_source(kind, T, S, page):
     """Flat, paged and planes calls take the positions of the call that returns
@@ -871,6 +871,33 @@ def test_paged_selection_without_scores_matches_oracle(T, Hi):
     torch.cuda.synchronize()
     ref, _ = _oracle(d, topk)
     assert np.array_equal(np.sort(got.cpu().numpy(), axis=1), np.sort(ref, axis=1))
+
+
+# on both sides of the rule that says whether the estimate kernel prepares K itself
+@pytest.mark.parametrize("T,Hi,S", [(2, 64, 32768), (2, 64, 32769), (4, 48, 16384), (4, 48, 16385), (5, 32, 21845),
+                                    (6, 16, 21846), (8, 64, 16384), (8, 64, 16385), (7, 48, 16385), (4, 32, 40000)])
+def test_selection_without_scores_where_k_is_prepared_ahead(T, Hi, S):
+    """The same sets from a flat and a paged cache as from prepared planes."""
+    from dsa_amd import prepare_k, run_indexer_and_topk_paged
+    page, topk = 64, 1500
+    d = _full_range(workloads.indexer_inputs(T=T, Hi=Hi, S=S, seed=Hi + T), torch.Generator().manual_seed(S))
+    d["causal_limit"] = torch.arange(S - 40 * T, S, 40, dtype=torch.int32)
+    d["causal_limit"][0] = topk + 3
+    n_pages = -(-S // page)
+    codes, scale = torch.zeros(n_pages * page, 128, dtype=torch.uint8), torch.zeros(n_pages * page)
+    codes[:S], scale[:S] = d["k_idx"].view(torch.uint8), d["k_scale"]
+    cache = torch.cat([codes.view(n_pages, -1), scale.view(n_pages, -1).view(torch.uint8)], dim=1).contiguous().to(DEV)
+    pages = torch.arange(n_pages, dtype=torch.int32, device=DEV)
+    g = workloads.to_device(d, DEV)
+    rest = (g["weights"], g["causal_limit"], topk)
+    print(f"K prepared ahead T={T} Hi={Hi} S={S}", flush=True)
+    want = run_indexer_and_topk(g["q_idx"], None, None, *rest, k_planes=prepare_k(g["k_idx"], g["k_scale"]))
+    flat = run_indexer_and_topk(g["q_idx"], g["k_idx"], g["k_scale"], *rest)
+    paged = run_indexer_and_topk_paged(g["q_idx"], cache, pages, S, *rest)
+    exact = run_indexer_and_topk(g["q_idx"], g["k_idx"], g["k_scale"], *rest, return_scores=True)[0]
+    torch.cuda.synchronize()
+    for name, x in (("flat", flat), ("paged", paged), ("exact", exact)):
+        assert torch.equal(x, want), name
 
 
 def _estimates(q, k, k_scale, w, topk):
