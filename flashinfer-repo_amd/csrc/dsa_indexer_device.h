@@ -102,14 +102,27 @@ __device__ __forceinline__ int magnitude_bound(uint32_t top) {
   return top == 0x7f ? (15 << 14) : e4m3_x(top);
 }
 
-// Wave-wide largest code & 0x7f of the 32 codes a lane holds in w[8].
+// Lane 63 gets the wave's largest value.
+__device__ __forceinline__ uint32_t wave_max_last(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
+}
+
+// Wave-wide largest code & 0x7f of the 32 codes a lane holds in w[8]: two bytes of
+// a dword at a time.
 __device__ __forceinline__ uint32_t wave_top_code(const uint32_t (&w)[8]) {
-  uint32_t mc = 0;
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  u16x2 m = {0, 0};
 #pragma unroll
-  for (int i = 0; i < 32; ++i) mc = max(mc, (w[i >> 2] >> (8 * (i & 3))) & 0x7fu);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mc = max(mc, (uint32_t)__shfl_xor((int)mc, o));
-  return __builtin_amdgcn_readfirstlane(mc);
+  for (int i = 0; i < 8; ++i) {
+    m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, w[i] & 0x007f007fu));
+    m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, (w[i] >> 8) & 0x007f007fu));
+  }
+  return __builtin_amdgcn_readlane(wave_max_last(max((uint32_t)m[0], (uint32_t)m[1])), 63);
 }
 
 // Plane `byte` of the LUT words v[32] of a lane's 2 x 16 codes (negated: the

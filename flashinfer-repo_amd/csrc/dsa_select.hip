@@ -203,15 +203,12 @@ __global__ __launch_bounds__(kEstWaves * 64, SRC == kPrepared ? 2 : 1) void dsa_
 #pragma unroll
       for (int j = 0; j < 2; ++j)
         n2 += sum_squares8(r.h[j][0], r.h[j][1]) + sum_squares8(r.h[j][2], r.h[j][3]);
-      n2 += __shfl_xor(n2, 16);
-      n2 += __shfl_xor(n2, 32);
+      n2 = sum_lane_groups(n2);
       const int s = blk * 16 + c;
       float cs = r.cs;
       if constexpr (SRC == kFlat) cs = s < p.S ? p.k_scale[s] * 0x1p-18f : 0.f;
-      uint32_t nb = position_norm_bits(cs, n2);
-#pragma unroll
-      for (int o = 8; o > 0; o >>= 1) nb = max(nb, (uint32_t)__shfl_xor((int)nb, o));
-      if (lane == 0) p.k_max[blk] = (int32_t)(nb << kMaxXBits);
+      const uint32_t nb = wave_max_last(position_norm_bits(cs, n2));
+      if (lane == 63) p.k_max[blk] = (int32_t)(nb << kMaxXBits);
       if (g == 0 && s < p.S) p.k_cs[s] = cs;
       if constexpr (SRC == kPaged) {
         uint8_t *dst = p.k_codes + (int64_t)blk * kCodeBlockBytes + kvo;
@@ -423,16 +420,6 @@ __device__ __forceinline__ float row_sum_last(float v) {
 __device__ __forceinline__ float rows_sum_last(float v) {
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xa, 0xf, false));
   return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xc, 0xf, false));
-}
-
-// Lane 63 gets the wave's largest value.
-__device__ __forceinline__ uint32_t wave_max_last(uint32_t v) {
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));
-  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
 }
 
 // Exclusive prefix sums of (a, b) over the 1024 threads of the block; the
