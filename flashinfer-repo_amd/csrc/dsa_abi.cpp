@@ -75,8 +75,9 @@ void choose_splits(int64_t T, int64_t H, int64_t K, int32_t requested, int32_t *
     const int64_t tiles = ceil_div(K, dsa::kKeysPerTile);
     int64_t max_s;
     // the four-wave layout while it gets at least 2 splits (at least 4 for
-    // multiples of 8 groups, whose four-wave ring layout is faster at 2:
-    // H=128 T=16 32 us with 8 splits against 36.8 us)
+    // multiples of 8 groups: with its own 8 to 13 splits their four-wave ring
+    // layout is faster than that with 2, or as fast: H=128 T=9 27.5 us against 29.4,
+    // T=13 29.1 against 30.6, T=16 30.3 against 29.9)
     if (groups % 2 != 0 || Tn * groups <= dsa::kNumCU / (groups % 8 == 0 ? 4 : 2)) {
       // four-wave layout, T x S x groups workgroups within one round
       S = dsa::kNumCU / (Tn * groups);

@@ -484,7 +484,8 @@ constexpr int kMaxOpen = 512;
 // (narrow_open; rows past 8192 positions only: the shorter ones' kernel takes
 // 0.2 us longer with it whatever the row), past that by two more radix passes,
 // which cost 4 us.  (64 rows of 32768 positions with a shared component four times
-// the noise took 1393 us when a crowded bin was scored whole, 55 now.)
+// the noise took 1393 us when a crowded bin was scored whole, 61 now; ordinary
+// rows take 56.)
 constexpr int kMaxBinOpen = 128;
 constexpr int kMaxNarrowed = 256;
 
@@ -1270,7 +1271,8 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_kernel(IndexerParam
 // bound (huge, tiny or non-finite weights or scales: all are open), the open
 // positions' exact scores replace their estimates in memory and the row is
 // selected from once more -- by this one workgroup: 64 rows of 32768
-// positions all tied at 0 take 490 us, of which a third are one same row 216.
+// positions all tied at 0 take 471 us, of which a third are one same row 222 (115
+// and 83 with every score from the score kernel).
 template <int EPT>
 __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_estimates_kernel(IndexerParams p) {
   constexpr int KEYS = EPT * kTopkThreads;
@@ -1331,7 +1333,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_idx_topk_estimates_kernel(In
 // positions, ascending.  A chunk whose bound is not safe, or too many of whose
 // scores lie within the bound of the k-th, lists its k largest, by the exact
 // scores of those.  2 rows of 131071 positions, top-k
-// 2048: chunks 17 us, lists 20, against 235 for the four passes over exact
+// 2048: chunks 17 us, lists 17, against 235 for the four passes over exact
 // scores (one workgroup re-reading the row, its last pass uncoalesced).
 
 // The chunk's marked keys (of its first n places) as its list.

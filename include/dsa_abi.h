@@ -288,7 +288,9 @@ int dsa_indexer_topk(const dsa_indexer_args *args, void *stream);
  * num_positions read as zeros), into a planes buffer laid out for
  * k_planes_capacity positions.  After an append, re-preparing the appended
  * positions keeps the planes current; calls of dsa_indexer_topk with those
- * planes give the same bits as calls that prepare K themselves.
+ * planes give the same bits as calls that prepare K themselves.  The layout of
+ * a planes buffer belongs to the library that wrote it: prepare it again from
+ * the K cache rather than reading one that another build has saved.
  */
 typedef struct dsa_indexer_k_prepare_args {
   const uint8_t *k_idx;     /* [num_positions, 128] e4m3fn codes, or NULL (paged) */
